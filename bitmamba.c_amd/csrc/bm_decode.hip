@@ -14,9 +14,9 @@
 //
 // Every block recomputes the RMSNorm/int8 prologue of its input.  Its
 // critical path is the sequential sum of squares (four fp32 chains,
-// src/kernel.c:77-89): the chains run from registers of one wave, one
-// dependent add per element, while the block's weight rows are already in
-// flight.  All elementwise prologue work runs on register-resident copies of
+// src/kernel.c:77-89): wave j runs chain j with chain_wave (bm_dev.h), or
+// wave 0 all four in turn at K = 1024 and in the LM head, while the block's
+// weight rows are already in flight.  All elementwise prologue work runs on register-resident copies of
 // the input.  Kernel boundaries order the phases; no grid-wide fences.
 #include <type_traits>
 
@@ -37,50 +37,28 @@ constexpr int kDoneArmed = 1, kDoneStopped = 2;
 __device__ __forceinline__ bool is_end_token(int t) { return t == 50256 || t == 0; }
 constexpr int kHist = 256;
 
-__device__ __forceinline__ float silu_r(float x) {
-  return cr_divf(x, __fadd_rn(1.0f, libm::expf_glibc(-x)));
+// the libm tables, in device memory or copied to LDS
+struct LibmTabs {
+  uint64_t exp2[32];
+  double invc[16], logc[16];
+};
+// the copy's word i (of 64), lane by lane
+__device__ __forceinline__ uint64_t libm_tab_word(int i) {
+  const uint64_t* src = i < 32   ? libm::kExp2Tab + i
+                        : i < 48 ? (const uint64_t*)libm::kLogInvC + (i - 32)
+                                 : (const uint64_t*)libm::kLogC + (i - 48);
+  return *src;
 }
 
-__device__ __forceinline__ float softplus_r(float x) {
+__device__ __forceinline__ float silu_r(float x, const uint64_t* exp2 = libm::kExp2Tab) {
+  return cr_divf(x, __fadd_rn(1.0f, libm::expf_tab(-x, exp2)));
+}
+
+__device__ __forceinline__ float softplus_r(float x, const uint64_t* exp2 = libm::kExp2Tab,
+                                            const double* invc = libm::kLogInvC,
+                                            const double* logc = libm::kLogC) {
   if (x > 20.0f) return x;
-  return libm::logf_glibc(__fadd_rn(1.0f, libm::expf_glibc(x)));
-}
-
-// ---------------------------------------------------------------------------
-// Sum of squares: four sequential chains
-// ---------------------------------------------------------------------------
-
-// other K: one lane per chain over LDS, two 32-value buffers alternating
-__device__ __forceinline__ void add32(float& s, const float4 (&b)[8]) {
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    s = __fadd_rn(s, b[u].x);
-    s = __fadd_rn(s, b[u].y);
-    s = __fadd_rn(s, b[u].z);
-    s = __fadd_rn(s, b[u].w);
-  }
-}
-
-__device__ __forceinline__ void load32(float4 (&b)[8], const float* __restrict__ c) {
-#pragma unroll
-  for (int u = 0; u < 8; ++u) b[u] = *(const float4*)(c + 4 * u);
-}
-
-__device__ __forceinline__ float chain_lds(const float* __restrict__ c, int len) {
-  float s = 0.0f;
-  int i = 0;
-  if (len >= 64) {
-    float4 A[8], B[8];
-    load32(A, c);
-    for (; i + 64 <= len; i += 64) {
-      load32(B, c + i + 32);
-      add32(s, A);
-      if (i + 96 <= len) load32(A, c + i + 64);
-      add32(s, B);
-    }
-  }
-  for (; i < len; ++i) s = __fadd_rn(s, c[i]);
-  return s;
+  return libm::logf_tab(__fadd_rn(1.0f, libm::expf_tab(x, exp2)), invc, logc);
 }
 
 // ---------------------------------------------------------------------------
@@ -99,7 +77,7 @@ __device__ __forceinline__ void stage_load(float4 (&st)[C], const float* __restr
 }
 
 struct Lds {
-  float* sq;      // [4][stride] squares, chain-major (padded per segment)
+  float* sq;      // [4][stride] squares, chain-major (chain_wave's layout)
   uint32_t* nib;  // [K/4] split-nibble activations
   int8_t* q8;     // [K] int8 activations
   int* slices;    // [S] sum of int8 per 1024-column slice
@@ -107,13 +85,19 @@ struct Lds {
   int stride;
 };
 
+// floats of one chain's squares: room for both chain layouts
+__host__ __device__ inline int sq_floats(int K) {
+  const int a = chain_floats(chain_elems(K)), b = sq_stride_of(K);
+  return a > b ? a : b;
+}
+
 __host__ __device__ inline size_t lds_bytes(int K) {
-  return 16 * (size_t)sq_stride_of(K) + 2 * (size_t)K + 4 * (size_t)((K + 1023) / 1024) + 16 + 128;
+  return 16 * (size_t)sq_floats(K) + 2 * (size_t)K + 4 * (size_t)((K + 1023) / 1024) + 16 + 128;
 }
 
 __device__ __forceinline__ Lds lds_carve(uint8_t* base, int K) {
   Lds l;
-  l.stride = sq_stride_of(K);
+  l.stride = sq_floats(K);
   l.sq = (float*)base;
   l.nib = (uint32_t*)(l.sq + 4 * l.stride);
   l.q8 = (int8_t*)(l.nib + K / 4);
@@ -122,47 +106,34 @@ __device__ __forceinline__ Lds lds_carve(uint8_t* base, int K) {
   return l;
 }
 
+// the four chain sums in bc[0..3], combined as the reference does:
+// 1/sqrtf(((s0+s1)+s2)+s3)/K + 1e-6f) (src/kernel.c:89-91)
+__device__ __forceinline__ float sum_chains(const float* bc) {
+  return __fadd_rn(__fadd_rn(__fadd_rn(bc[0], bc[1]), bc[2]), bc[3]);
+}
+
 // rms = 1/sqrtf(sum_sq/K + 1e-6f) with the sequential four-chain sum
-// (src/kernel.c:77-91)
+// (src/kernel.c:77-91), wave j running chain j.  A chain's K/4 elements are
+// padded with zeros (which add nothing) to 64 * E.
 template <int C>
 __device__ float pro_rms(const float4 (&xv)[C], int K, const Lds& l) {
-  const int tid = threadIdx.x, nt = blockDim.x, n4 = K >> 2;
-  const bool regs = chain_in_regs(K);
-  const int E = K >> 6;
+  constexpr int E = 4 * C;  // K <= 1024 * C
+  static_assert(C == 1 || C == 2 || C == 4 || C == 8, "chain_elems");
+  const int tid = threadIdx.x, nt = blockDim.x, wave = tid >> 6;
 #pragma unroll
   for (int i = 0; i < C; ++i) {
-    const int c = tid + i * nt;
-    if (c < n4) {
-      const int e = c + (regs ? 4 * (c / E) : 0);
-      l.sq[e] = __fmul_rn(xv[i].x, xv[i].x);
-      l.sq[l.stride + e] = __fmul_rn(xv[i].y, xv[i].y);
-      l.sq[2 * l.stride + e] = __fmul_rn(xv[i].z, xv[i].z);
-      l.sq[3 * l.stride + e] = __fmul_rn(xv[i].w, xv[i].w);
-    }
+    const int c = tid + i * nt;  // C * nt = 64 * E: xv is zero past K
+    const int e = c + chain_pad(E) * (c / E);
+    l.sq[e] = __fmul_rn(xv[i].x, xv[i].x);
+    l.sq[l.stride + e] = __fmul_rn(xv[i].y, xv[i].y);
+    l.sq[2 * l.stride + e] = __fmul_rn(xv[i].z, xv[i].z);
+    l.sq[3 * l.stride + e] = __fmul_rn(xv[i].w, xv[i].w);
   }
   __syncthreads();
-  if (tid < 64) {
-    float cs = 0.0f;
-    if (regs) {
-      if (K == 1024)
-        cs = chain_regs<16>(l.sq, l.stride, tid);
-      else if (K == 2048)
-        cs = chain_regs<32>(l.sq, l.stride, tid);
-      else
-        cs = chain_regs<64>(l.sq, l.stride, tid);
-    } else if ((tid & 15) == 15) {
-      cs = chain_lds(l.sq + (tid >> 4) * l.stride, n4);
-    }
-    // lanes 15, 31, 47, 63 hold the chain sums: ((s0+s1)+s2)+s3
-    const float s0 = __shfl(cs, 15, 64), s1 = __shfl(cs, 31, 64);
-    const float s2 = __shfl(cs, 47, 64), s3 = __shfl(cs, 63, 64);
-    if (tid == 0) {
-      const float sum = __fadd_rn(__fadd_rn(__fadd_rn(s0, s1), s2), s3);
-      l.bc[0] = cr_divf(1.0f, cr_sqrtf(__fadd_rn(cr_divf(sum, (float)K), 1e-6f)));
-    }
-  }
+  const float cs = chain_wave_lds<E>(l.sq + wave * l.stride, 0.0f);
+  if ((tid & 63) == 0) l.bc[wave] = cs;
   __syncthreads();
-  return l.bc[0];
+  return cr_divf(1.0f, cr_sqrtf(__fadd_rn(cr_divf(sum_chains(l.bc), (float)K), 1e-6f)));
 }
 
 __device__ __forceinline__ float4 scale4(const float4& x, float rms, const float4& g) {
@@ -258,48 +229,62 @@ __device__ float pro_quant(const float4 (&xv)[C], const float4 (&gv)[C], float r
 // scale_x.
 //   PRENORM: x first becomes (x * rms(x)) * g_pre (the final norm).
 // ---------------------------------------------------------------------------
-template <int G>
+template <int G, bool ONE>
 __device__ __forceinline__ void put_squares(const float4 (&v)[G], const Lds& l) {
-  constexpr int E = 1024 * G / 64;
-  // column 4e + j is element e of chain j (segments of E elements padded by
-  // 4 floats); the thread's elements G*t .. G*t+G-1 lie in one segment
+  // ONE: the layout of chain_regs, else of chain_wave
+  constexpr int E = ONE ? 16 * G : 4 * G, PAD = ONE ? 4 : chain_pad(E);
+  // column 4e + j is element e of chain j; the thread's elements G*t ..
+  // G*t+G-1 lie in one lane's segment
   const int e = G * (int)threadIdx.x;
-  const int pe = e + 4 * (e / E);
+  float* __restrict__ d = l.sq + e + PAD * (e / E);
+  if constexpr (G == 4) {
+    *(float4*)d = make_float4(__fmul_rn(v[0].x, v[0].x), __fmul_rn(v[1].x, v[1].x),
+                              __fmul_rn(v[2].x, v[2].x), __fmul_rn(v[3].x, v[3].x));
+    *(float4*)(d + l.stride) = make_float4(__fmul_rn(v[0].y, v[0].y), __fmul_rn(v[1].y, v[1].y),
+                                           __fmul_rn(v[2].y, v[2].y), __fmul_rn(v[3].y, v[3].y));
+    *(float4*)(d + 2 * l.stride) =
+        make_float4(__fmul_rn(v[0].z, v[0].z), __fmul_rn(v[1].z, v[1].z),
+                    __fmul_rn(v[2].z, v[2].z), __fmul_rn(v[3].z, v[3].z));
+    *(float4*)(d + 3 * l.stride) =
+        make_float4(__fmul_rn(v[0].w, v[0].w), __fmul_rn(v[1].w, v[1].w),
+                    __fmul_rn(v[2].w, v[2].w), __fmul_rn(v[3].w, v[3].w));
+  } else {
 #pragma unroll
-  for (int k = 0; k < G; ++k) {
-    l.sq[pe + k] = __fmul_rn(v[k].x, v[k].x);
-    l.sq[l.stride + pe + k] = __fmul_rn(v[k].y, v[k].y);
-    l.sq[2 * l.stride + pe + k] = __fmul_rn(v[k].z, v[k].z);
-    l.sq[3 * l.stride + pe + k] = __fmul_rn(v[k].w, v[k].w);
+    for (int k = 0; k < G; ++k) {
+      d[k] = __fmul_rn(v[k].x, v[k].x);
+      d[l.stride + k] = __fmul_rn(v[k].y, v[k].y);
+      d[2 * l.stride + k] = __fmul_rn(v[k].z, v[k].z);
+      d[3 * l.stride + k] = __fmul_rn(v[k].w, v[k].w);
+    }
   }
 }
 
-// rms = 1/sqrtf(sum/K + 1e-6f) from the squares in LDS; wave 0 runs the
-// chains, the result is broadcast through LDS (src/kernel.c:77-91); the
-// other waves run `idle` meanwhile
 struct NoWork {
   __device__ void operator()() const {}
 };
 
-template <int G, typename F = NoWork>
+// rms = 1/sqrtf(sum/K + 1e-6f) from the squares in LDS (src/kernel.c:77-91):
+// wave j runs chain j, or (ONE) wave 0 all four while the other waves run
+// `idle`; every thread forms the result from the four sums
+template <int G, bool ONE, typename F = NoWork>
 __device__ __forceinline__ float chain_rms(const Lds& l, F&& idle = NoWork{}) {
-  constexpr int K = 1024 * G, E = K / 64;
+  constexpr int K = 1024 * G;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __syncthreads();
-  if (threadIdx.x >= 64) {
-    idle();
-  } else {
-    const float cs = chain_regs<E>(l.sq, l.stride, threadIdx.x);
-    const float s0 = lane_f32(cs, 15), s1 = lane_f32(cs, 31);
-    const float s2 = lane_f32(cs, 47), s3 = lane_f32(cs, 63);
-    if (threadIdx.x == 0) {
-      const float sum = __fadd_rn(__fadd_rn(__fadd_rn(s0, s1), s2), s3);
-      // sum / K with K a power of two: an exact scaling, rounded like the
-      // division
-      l.bc[0] = cr_divf(1.0f, cr_sqrtf(__fadd_rn(__fmul_rn(sum, 1.0f / K), 1e-6f)));
+  if constexpr (ONE) {
+    if (threadIdx.x >= 64) {
+      idle();
+    } else {
+      const float cs = chain_regs<16 * G>(l.sq, l.stride, lane);
+      if ((lane & 15) == 15) l.bc[lane >> 4] = cs;
     }
+  } else {
+    const float cs = chain_wave_lds<4 * G>(l.sq + wave * l.stride, 0.0f);
+    if (lane == 0) l.bc[wave] = cs;
   }
   __syncthreads();
-  return l.bc[0];
+  // sum / K with K a power of two: an exact scaling, rounded like the division
+  return cr_divf(1.0f, cr_sqrtf(__fadd_rn(__fmul_rn(sum_chains(l.bc), 1.0f / K), 1e-6f)));
 }
 
 // the thread's columns of the input and of the norm weights, loaded at
@@ -350,7 +335,7 @@ __device__ __forceinline__ float fast_rms(const float4 (&xv)[G], const Lds& l) {
   return cr_divf(1.0f, cr_sqrtf(__fadd_rn(__fmul_rn(s, 1.0f / K), 1e-6f)));
 }
 
-// idle: work for waves 1.. while wave 0 runs the first chain (the first
+// idle: work for waves 1.. while wave 0 runs the first chains (the first
 // fast-mode tree has no such window: they run it at once)
 template <int G, bool PRENORM, typename F = NoWork>
 __device__ float split_prologue(SplitIn<G, PRENORM>& in, const Lds& l, bool fast,
@@ -362,12 +347,16 @@ __device__ float split_prologue(SplitIn<G, PRENORM>& in, const Lds& l, bool fast
   float4 (&xv)[G] = in.xv;
   const float4 (&gv)[G] = in.gv;
   const float4 (&gp)[PRENORM ? G : 1] = in.gp;
+  // wave 0 alone runs the chains where that takes no longer (K = 1024: 4.52
+  // against 4.80 us per 255M in_proj launch) or the other waves have rows to
+  // issue meanwhile (the LM head: 11.7 against 12.4 us at K = 2048)
+  constexpr bool ONE = G == 1 || !std::is_same<std::decay_t<F>, NoWork>::value;
   float rms;
   if (fast) {
     if (threadIdx.x >= 64) idle();
     rms = fast_rms<G>(xv, l);
   } else {
-    put_squares<G>(xv, l);
+    put_squares<G, ONE>(xv, l);
     if constexpr (!std::is_same<std::decay_t<F>, NoWork>::value) {
       // waves 1.. issue their rows during the chain: the other inputs are
       // passed through an empty asm first (which waits for them now), so
@@ -382,7 +371,7 @@ __device__ float split_prologue(SplitIn<G, PRENORM>& in, const Lds& l, bool fast
           asm volatile("" : "+v"(in.gp[k].x), "+v"(in.gp[k].y), "+v"(in.gp[k].z), "+v"(in.gp[k].w));
       }
     }
-    rms = chain_rms<G>(l, idle);
+    rms = chain_rms<G, ONE>(l, idle);
   }
   if constexpr (PRENORM) {
     // final_feat = (x * rms) * norm_f (src/model.c:1225, src/kernel.c:93-103)
@@ -392,8 +381,8 @@ __device__ float split_prologue(SplitIn<G, PRENORM>& in, const Lds& l, bool fast
       __syncthreads();  // the first tree's sums are read before they are replaced
       rms = fast_rms<G>(xv, l);
     } else {
-      put_squares<G>(xv, l);
-      rms = chain_rms<G>(l);
+      put_squares<G, ONE>(xv, l);
+      rms = chain_rms<G, ONE>(l);
     }
   }
   // int8 quantization (src/kernel.c:93-128, 358-386)
@@ -637,7 +626,7 @@ __global__ __launch_bounds__(256) void k_rows_fused(const float* __restrict__ x,
     resid[it] = (MODE == 1 && u == 0 && g0 + wave + 4 * it < g1 && r < N) ? out[r] : 0.0f;
   }
 
-  const Lds l = lds_carve(lds, K);
+  const Lds l = lds_carve(lds, WP ? 1024 * C : K);
   float* const xn_out = b == 0 ? dr.xn : nullptr;
   int8_t* const xq_out = b == 0 ? dr.xq : nullptr;
   float scale_x;
@@ -660,8 +649,8 @@ __global__ __launch_bounds__(256) void k_rows_fused(const float* __restrict__ x,
       scale_x = pro_quant<C>(sx, sg, rms, K, l, xn_out, xq_out);
     }
   }
-  if (defer_rows && wave == 0) load_rows();
   if (b == 0 && tid == 0 && dr.scale) *dr.scale = scale_x;
+  if (defer_rows && wave == 0) load_rows();
   const float inv = inv_scale_of(scale_x, w_scale);
   uint32_t xa[P][16];
   int xsl[P], xsd[P];  // slice sums (after the reduction) or lane shares (before it)
@@ -1020,8 +1009,13 @@ __global__ __launch_bounds__(256) void k_inproj_ssm(const float* __restrict__ x,
   const float cw0 = a.cw[idx], cw1 = a.cw[a.di + idx], cw2 = a.cw[2 * a.di + idx];
   const float cw3 = a.cw[3 * a.di + idx], cbias = a.cb[idx], st0 = a.ssm[idx], Dc = a.D[idx];
   const float dtb = a.dt_bias[h], Ah = a.A[h];
+  // the tables of expf and logf, copied to LDS by wave 3: a lookup in device
+  // memory costs a cache miss in every launch, and the decay has three in a row
+  __shared__ LibmTabs s_libm;
+  uint64_t tab_word = 0;
+  if (wave == 3) tab_word = libm_tab_word(lane);
 
-  const Lds l = lds_carve(lds, K);
+  const Lds l = lds_carve(lds, WP ? 1024 * C : K);
   float scale_x;
   if constexpr (WP) {
     scale_x = split_prologue<C, false>(sin, l, fast != 0);
@@ -1053,6 +1047,7 @@ __global__ __launch_bounds__(256) void k_inproj_ssm(const float* __restrict__ x,
       if (u == 0 && r < kRowsCB) s_proj[r] = o;
     }
   }
+  if (wave == 3) ((uint64_t*)&s_libm)[lane] = tab_word;
   __syncthreads();
 
   // scalar_ssm_inner for the block's channels (src/kernel.c:34-70), its
@@ -1071,13 +1066,14 @@ __global__ __launch_bounds__(256) void k_inproj_ssm(const float* __restrict__ x,
     conv = __fadd_rn(conv, __fmul_rn(tap2, cw2));
     conv = __fadd_rn(conv, __fmul_rn(xin, cw3));
     if (!stopped) a.cs[(size_t)pos * a.di + idx] = xin;  // the oldest tap is overwritten
-    s_tail[c] = silu_r(conv);
+    s_tail[c] = silu_r(conv, s_libm.exp2);
   } else if (wave == 1 && lane < kCB) {
-    s_tail[kCB + lane] = silu_r(s_proj[lane]);
+    s_tail[kCB + lane] = silu_r(s_proj[lane], s_libm.exp2);
   } else if (wave == 2 && lane == 0) {
-    const float dt_val = softplus_r(__fadd_rn(s_proj[2 * kCB + 2], dtb));
+    const float dt_val = softplus_r(__fadd_rn(s_proj[2 * kCB + 2], dtb), s_libm.exp2, s_libm.invc,
+                                    s_libm.logc);
     s_tail[2 * kCB] = dt_val;
-    s_tail[2 * kCB + 1] = libm::expf_glibc(__fmul_rn(Ah, dt_val));
+    s_tail[2 * kCB + 1] = libm::expf_tab(__fmul_rn(Ah, dt_val), s_libm.exp2);
   }
   __syncthreads();
   if (tid < kCB && stopped) {

@@ -130,13 +130,6 @@ __device__ __forceinline__ int row_total_i32(int part, int xs_slice, int unit_ba
 }
 
 // ---------------------------------------------------------------------------
-// Sum of squares in the four sequential chains (src/kernel.c:77-89)
-// ---------------------------------------------------------------------------
-// chains held in registers (K/64 = E in {16, 32, 64}): lanes 16j..16j+15 of
-// wave 0 own chain j in segments of E consecutive elements; each lane adds
-// its segment to the running sum, which then moves one lane up the 16-lane
-// row (DPP row_shr:1).  After 16 rounds lane 16j+15 holds chain j's sum.
-// ---------------------------------------------------------------------------
 // Fast mode (opt-in, not the reference's bits): the sum of squares as one
 // balanced pairwise tree over the columns -- 16 consecutive columns per
 // leaf group, (((c0+c1)+(c2+c3))+((c4+c5)+(c6+c7)))+..., then the groups
@@ -174,7 +167,14 @@ __device__ __forceinline__ float tree_top(const float* w) {
   return __fadd_rn(__fadd_rn(w[0], w[1]), __fadd_rn(w[2], w[3]));
 }
 
-__host__ __device__ inline bool chain_in_regs(int K) { return K == 1024 || K == 2048 || K == 4096; }
+// ---------------------------------------------------------------------------
+// Sum of squares in the four sequential chains (src/kernel.c:77-89), all four
+// on one wave
+// ---------------------------------------------------------------------------
+// chains held in registers (K/64 = E in {16, 32, 64}): lanes 16j..16j+15 of
+// the wave own chain j in segments of E consecutive elements; each lane adds
+// its segment to the running sum, which then moves one lane up the 16-lane
+// row (DPP row_shr:1).  After 16 rounds lane 16j+15 holds chain j's sum.
 __host__ __device__ inline int sq_stride_of(int K) { return K / 4 + 68; }
 
 template <int E>
@@ -200,6 +200,150 @@ __device__ __forceinline__ float chain_regs(const float* __restrict__ sq, int st
                                                      0xf, 0xf, false));
   }
   return s;
+}
+
+// ---------------------------------------------------------------------------
+// The running fp32 sum of a chain of non-negative values (squares), with the
+// rounding of every single add kept, by one whole wave instead of one lane.
+//
+// Lane l holds elements E*l .. E*l+E-1.  While a running sum stays inside one
+// binade [2^e, 2^(e+1)), adding c moves its bit pattern by an integer that
+// depends on the pattern only through its lowest bit (ties round to even).  So
+// each lane runs its E adds twice, from an approximate start p (a prefix sum
+// in another order) and from the next float above it.  If both end in p's
+// binade and moved by the same integer d, the lane moves every start in the
+// binade by d, and the moves of consecutive lanes add up (a prefix sum of
+// integers).  The other lanes -- the sum leaves the binade, which happens
+// about log2(64) times after lane 0, or a tie makes the two moves differ,
+// about as often -- are added up again from their exact start, one after the
+// other.  At the end every lane's exact start and end are checked to lie in
+// the binade that was assumed for it (the map is monotone, so everything in
+// between then does too); if one does not, the chain is added up in turn.
+// Infinities and NaNs (exponent 255) are always added up.  Zeros at the end
+// leave the sum as it is, so chains are padded with them.
+//
+// What bounds it: one wave's instruction issue, ~4.7 cycles per dependent add
+// (ten lanes added up again cost about as much as everything else).  A chain
+// of normal squares takes ~1450 / 2200 cycles at 512 / 1024 elements (K =
+// 2048 / 4096), against ~2500 / 5000 for one lane adding in turn; at 256 (K =
+// 1024) both take ~1250, and chain_regs stays.  Per launch of the 1B decode:
+// out_proj 5.78 -> 4.57 us, in_proj 5.61 -> 5.34; the greedy step 0.2895 ->
+// 0.260 ms.
+// ---------------------------------------------------------------------------
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ int dpp_or0(int v) {  // lanes without a source get 0
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+
+// inclusive prefix sums over the wave; in fp32 in any order of adds
+__device__ __forceinline__ float wave_scan_f32(float v) {
+  v = __fadd_rn(v, __int_as_float(dpp_or0<0x111>(__float_as_int(v))));
+  v = __fadd_rn(v, __int_as_float(dpp_or0<0x112>(__float_as_int(v))));
+  v = __fadd_rn(v, __int_as_float(dpp_or0<0x114>(__float_as_int(v))));
+  v = __fadd_rn(v, __int_as_float(dpp_or0<0x118>(__float_as_int(v))));
+  v = __fadd_rn(v, __int_as_float(dpp_or0<0x142, 0xa>(__float_as_int(v))));
+  return __fadd_rn(v, __int_as_float(dpp_or0<0x143, 0xc>(__float_as_int(v))));
+}
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
+  v += (uint32_t)dpp_or0<0x111>((int)v);
+  v += (uint32_t)dpp_or0<0x112>((int)v);
+  v += (uint32_t)dpp_or0<0x114>((int)v);
+  v += (uint32_t)dpp_or0<0x118>((int)v);
+  v += (uint32_t)dpp_or0<0x142, 0xa>((int)v);
+  return v + (uint32_t)dpp_or0<0x143, 0xc>((int)v);
+}
+
+// c: the lane's E elements; start: the sum so far (uniform, >= 0 or NaN);
+// returns the sum after all 64 * E elements (uniform).  The first HEAD lanes
+// are added up in turn at once, each handing its sum to the next (DPP
+// row_shr:1), since the sum doubles often there: worth it for short lanes
+// (1B in_proj launch, E = 8: 5.34 us with HEAD = 8, 5.48 with 4, 5.51 with 1;
+// out_proj, E = 16: 4.86, 4.77, 4.58).
+template <int E>
+__device__ __forceinline__ float chain_wave(const float (&c)[E], float start) {
+  constexpr uint32_t kBinade = 0x00800000u;  // patterns per binade
+  constexpr int HEAD = E <= 8 ? 8 : 1;
+  const int lane = threadIdx.x & 63;
+  float t[E];
+#pragma unroll
+  for (int k = 0; k < E; ++k) t[k] = c[k];
+#pragma unroll
+  for (int w = E / 2; w >= 1; w /= 2)
+#pragma unroll
+    for (int k = 0; k < w; ++k) t[k] = __fadd_rn(t[k], t[k + w]);
+  // the approximate sum before the lane (DPP wave_shr:1 of the prefix sums)
+  const float before = __int_as_float(dpp_or0<0x138>(__float_as_int(wave_scan_f32(t[0]))));
+  float head = start;
+#pragma unroll
+  for (int h = 0; h < HEAD; ++h) {
+    if (h) head = __int_as_float(dpp_or0<0x111>(__float_as_int(head)));
+#pragma unroll
+    for (int k = 0; k < E; ++k) head = __fadd_rn(head, c[k]);
+  }
+  head = lane_f32(head, HEAD - 1);
+  const float p = __fadd_rn(head, __fsub_rn(before, lane_f32(before, HEAD)));
+  const uint32_t pb = __float_as_uint(p);
+  float a = p, b = __uint_as_float(pb + 1);
+#pragma unroll
+  for (int k = 0; k < E; ++k) {
+    a = __fadd_rn(a, c[k]);
+    b = __fadd_rn(b, c[k]);
+  }
+  const uint32_t ab = __float_as_uint(a), bb = __float_as_uint(b);
+  const bool moves = (pb ^ bb) < kBinade && pb < 0x7f800000u && bb == ab + 1 && lane >= HEAD;
+  const uint32_t d = moves ? ab - pb : 0;
+  const uint32_t sum = wave_scan_u32(d);  // moves up to and including the lane
+
+  // the exact sum after a lane is r + sum; r changes at the lanes added up
+  // (all lanes add, the one whose turn it is counts)
+  uint32_t cur = __float_as_uint(head) + sum, to = cur;
+  for (uint64_t left = __ballot(!moves) & (~0ull << HEAD); left;) {
+    const int l = __ffsll((unsigned long long)left) - 1;
+    left ^= 1ull << l;
+    float x = __uint_as_float(cur);
+#pragma unroll
+    for (int k = 0; k < E; ++k) x = __fadd_rn(x, c[k]);
+    cur = (uint32_t)__builtin_amdgcn_readlane((int)(__float_as_uint(x) - sum), l) + sum;
+    to = lane >= l ? cur : to;
+  }
+  const uint32_t from = to - d;
+  const bool off = moves && ((to ^ pb) >= kBinade || (from ^ pb) >= kBinade);
+  if (__ballot(off) == 0)
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)to, 63));
+  // a sum left the binade assumed for its lane: lane by lane
+  float x = head;
+#pragma unroll 1
+  for (int l = HEAD; l < 64; ++l) {
+#pragma unroll
+    for (int k = 0; k < E; ++k) x = __fadd_rn(x, c[k]);
+    x = lane_f32(x, l);
+  }
+  return x;
+}
+
+// LDS layout of a chain for chain_wave: lane l's E elements start at float
+// (E + pad) * l, padded by 4 floats where E > 4 so that 16 lanes' 16-byte
+// reads fall on different banks
+__host__ __device__ constexpr int chain_pad(int E) { return E > 4 ? 4 : 0; }
+__host__ __device__ constexpr int chain_floats(int E) { return 64 * (E + chain_pad(E)); }
+// elements per lane for chains of K/4 elements, K <= 8192
+__host__ __device__ inline int chain_elems(int K) {
+  return K <= 1024 ? 4 : (K <= 2048 ? 8 : (K <= 4096 ? 16 : 32));
+}
+
+template <int E>
+__device__ __forceinline__ float chain_wave_lds(const float* __restrict__ chain, float start) {
+  const float* __restrict__ src = chain + (threadIdx.x & 63) * (E + chain_pad(E));
+  float c[E];
+#pragma unroll
+  for (int u = 0; u < E / 4; ++u) {
+    const float4 q = *(const float4*)(src + 4 * u);
+    c[4 * u] = q.x;
+    c[4 * u + 1] = q.y;
+    c[4 * u + 2] = q.z;
+    c[4 * u + 3] = q.w;
+  }
+  return chain_wave<E>(c, start);
 }
 
 __device__ __forceinline__ float inv_scale_of(float scale_x, float w_scale) {

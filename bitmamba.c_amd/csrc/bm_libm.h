@@ -48,7 +48,8 @@ inline constexpr uint64_t kExp2Tab[32] = {
     0x3fefa4afa2a490daull, 0x3fefd0765b6e4540ull,
 };
 
-BM_HD float expf_glibc(float x) {
+// tab: kExp2Tab or a copy of it
+BM_HD float expf_tab(float x, const uint64_t* tab) {
   // special cases (selected at the end, no branches): overflow above
   // ~88.72, underflow to 0 below ~-103.97, NaN passes through
   const bool nan = x != x;
@@ -65,7 +66,7 @@ BM_HD float expf_glibc(float x) {
   const uint64_t ki = u64_of(kd);
   kd -= Shift;
   const double r = __builtin_fma(InvLn2N, xd, -kd);
-  uint64_t t = kExp2Tab[ki % 32];
+  uint64_t t = tab[ki % 32];
   t += ki << (52 - 5);
   const double s = dbl_of(t);
   const double z = __builtin_fma(C0, r, C1);
@@ -78,6 +79,7 @@ BM_HD float expf_glibc(float x) {
   res = ovf ? __builtin_inff() : res;
   return nan ? x : res;
 }
+BM_HD float expf_glibc(float x) { return expf_tab(x, kExp2Tab); }
 
 // (1/c, log c) for the 16 subintervals of [0x3f330000, 2 * 0x3f330000)
 inline constexpr double kLogInvC[16] = {
@@ -93,7 +95,8 @@ inline constexpr double kLogC[16] = {
     0x1.526e57720db08p-3, 0x1.bc2860d22477p-3, 0x1.1058bc8a07ee1p-2, 0x1.4043057b6ee09p-2,
 };
 
-BM_HD float logf_glibc(float x) {
+// invc_tab, logc_tab: kLogInvC and kLogC or copies of them
+BM_HD float logf_tab(float x, const double* invc_tab, const double* logc_tab) {
   // special inputs are handled by selects after the main path: 1 -> 0,
   // +-0 -> -inf, +inf -> +inf, negative or NaN -> NaN; subnormals are
   // normalized first
@@ -109,7 +112,7 @@ BM_HD float logf_glibc(float x) {
   const int i = (int)((tmp >> (23 - 4)) % 16);
   const int k = (int32_t)tmp >> 23;
   const uint32_t iz = ix - (tmp & (0x1ffu << 23));
-  const double invc = kLogInvC[i], logc = kLogC[i];
+  const double invc = invc_tab[i], logc = logc_tab[i];
   const double z = (double)flt_of(iz);
   // log(x) = log1p(z/c - 1) + log(c) + k*Ln2
   const double r = __builtin_fma(z, invc, -1.0);
@@ -126,6 +129,7 @@ BM_HD float logf_glibc(float x) {
   }
   return ix0 == 0x3f800000u ? 0.0f : res;
 }
+BM_HD float logf_glibc(float x) { return logf_tab(x, kLogInvC, kLogC); }
 
 }  // namespace libm
 }  // namespace bm

@@ -1,0 +1,60 @@
+"""The wave-parallel running sum of squares (bm_dev.h, chain_wave): rows that
+would show any difference from the one-by-one fp32 sum, through every kernel
+that uses it, bit-exact against the oracle.  Widths at the edges of the
+elements-per-lane classes, padded chains and the largest of each."""
+import numpy as np
+import pytest
+
+import native
+from native import bh, same_bits
+
+pytestmark = pytest.mark.gpu
+DB = bh.DeviceBuffer
+
+
+def rows_for(n, seed):
+    r = np.random.default_rng(seed)
+    c = (n + 3) // 4
+    # sums to 2^24 - 1, then adds of 1/4 that each round away: the sum stays
+    # below 2^24 while any sum in another order passes it
+    stuck = np.full(c, 0.5)
+    stuck[:4] = [4095.0, 90.0, 9.0, 3.0]
+    # the same one add later in the chain, inside a lane
+    late = np.roll(stuck, min(c - 4, c // 2 + 1))
+    late[: min(c - 4, c // 2 + 1)] = 0.0
+    rows = [
+        r.standard_normal(n) * np.exp(r.standard_normal(n)),
+        np.where(r.random(n) < 0.02, 4096.0, 1.0),   # ties at half an ulp
+        np.ldexp(1.0, r.integers(-20, 20, n)),
+        r.integers(-3, 4, n).astype(np.float64),     # sums that hit powers of two
+        r.standard_normal(n) * 1e-23,                # denormal squares
+        np.zeros(n),
+        np.where(np.arange(n) == n - 1, 3.0, 0.0),
+        np.where(np.arange(n) == n // 2, 1e20, r.standard_normal(n)),  # inf from there on
+        np.repeat(stuck, 4)[:n],
+        np.repeat(late, 4)[:n],
+        np.geomspace(1e-6, 1e6, n),                  # a new binade every few adds
+    ]
+    return np.ascontiguousarray(np.stack(rows).astype(np.float32))
+
+
+@pytest.mark.parametrize("K", [64, 1024, 1088, 2048, 2112, 4096, 4160, 8192])
+def test_one_token_prologue(hip, K):
+    """bm_hip_bitlinear_dev at one token: the fused row kernel's prologue."""
+    N = 128
+    packed = bh.synth_ternary(5, 1, N, K, bh.SYNTH_P0_40)
+    g = (np.random.default_rng(K).standard_normal(K) * 0.02).astype(np.float32)
+    x = rows_for(K, K)
+    dg, dw = DB.from_array(g), DB.from_array(packed)
+    for i in range(x.shape[0]):
+        print("one token K=%d row %d" % (K, i), flush=True)
+        dx, do, dq, ds = DB.from_array(x[i]), DB(4 * N), DB(K), DB(4)
+        da = DB(hip.bm_hip_act_bytes(1, K))
+        bh.check(hip.bm_hip_bitlinear_dev(dx.ptr, 1, K, dg.ptr, dw.ptr, N, 0.02, 1, do.ptr, dq.ptr,
+                                          K, ds.ptr, da.ptr, None), "bitlinear")
+        hip.bm_hip_synchronize()
+        on, oq, osc, _ = native.orc_quantize_rows(x[i:i + 1], g)
+        np.testing.assert_array_equal(dq.download(K, np.int8), oq[0])
+        same_bits(ds.download(1, np.float32), osc, "scale row %d" % i)
+        ref, _, _ = native.orc_bitlinear(x[i:i + 1], packed, N, K, 0.02, g)
+        same_bits(do.download(N, np.float32), ref[0], "out row %d" % i)
