@@ -12,15 +12,19 @@
 //                 lowest threshold the extraction can use (the histogram's
 //                 last bucket, or the min_p threshold), a superset of the
 //                 candidates.
+//   k_samp_probs  (no top-k) the probabilities, and per value bucket their
+//                 count and sum.
 // k_sample then runs the rest on one 1024-thread block: the cutoff bucket,
 // the candidates filtered from the pre-candidate lists in order, selection,
 // softmax, sorting and the draw, the step bookkeeping and the next token's
 // embedding.  (Pass 2 and this in one kernel, with a block counter and
 // device-scope fences handing over to the last block, measured 32 us per
 // token against about 14 for the two launches.)
-// The steps whose result depends on their order stay sequential on one
-// thread, in the reference's order: the heap selections (their array order
-// feeds the sums), every double sum, and the CDF walk.  Sorting is stable
+// With top-k, the steps whose result depends on their order stay sequential on
+// one thread, in the reference's order: the heap selection (its array order
+// feeds the sums), every double sum, and the CDF walk.  Without top-k the same
+// sums in any order decide nearly every draw (draw_parallel); the sequential
+// steps remain for the draws they leave open.  Sorting is stable
 // like glibc's qsort (a merge sort for these sizes), keyed on the value.
 // Float-to-int bucket indices follow x86 cvttss2si (out of range -> INT_MIN).
 #include "bm_common.h"
@@ -63,21 +67,44 @@ constexpr int kMaxVocab = 256000;  // MAX_VOCAB of the loader (src/bitmamba.h:55
 // vocabulary segment of each front block: a multiple of 4 entries
 __host__ __device__ __forceinline__ int front_seg(int V) { return ((V + kFront - 1) / kFront + 3) & ~3; }
 
+// Buckets of the draw without top-k: a probability's leading bits (sign,
+// exponent, 4 bits of the mantissa), in value order; probabilities are <= 1
+constexpr int kPShift = 19;
+constexpr int kPBuckets = 2048;
+static_assert((0x3f800000u >> kPShift) < kPBuckets, "1.0f has a bucket");
+__device__ __forceinline__ int p_bucket(float v) {
+  return min((int)(__float_as_uint(v) >> kPShift), kPBuckets - 1);
+}
+
 // scratch: probs[V], pre[kFront * seg] (also the radix sort's second
-// buffer), pmax[kFront], pcnt[kFront], hist[kBuckets].  hist is zero
-// between calls: k_samp_scale clears it, and so does k_sample after use.
+// buffer), esum[kFront], psum[kFront], bsum[kPBuckets], pv[kFront * seg]
+// (beside pre: exp(logit - max), then the probability), bcnt[kPBuckets],
+// pmax[kFront], pcnt[kFront], hist[kBuckets].  hist is zero between calls:
+// k_samp_scale clears it, and so does k_sample after use.
 struct Scratch {
   Cand* probs;
   Cand* pre;
+  double* esum;
+  double* psum;
+  double* bsum;
+  float* pv;
+  int* bcnt;
   float* pmax;
   int* pcnt;
   int* hist;
 };
 __host__ __device__ __forceinline__ Scratch scratch_of(void* base, int V) {
   Scratch s;
-  s.probs = (Cand*)base;
-  s.pre = s.probs + V;
-  s.pmax = (float*)(s.pre + (size_t)kFront * front_seg(V));
+  // from the first 16-byte boundary, and an even number of 8-byte entries, so
+  // that pv starts on 16 bytes
+  s.probs = (Cand*)(((uintptr_t)base + 15) & ~(uintptr_t)15);
+  s.pre = s.probs + (V + 1) / 2 * 2;
+  s.esum = (double*)(s.pre + (size_t)kFront * front_seg(V));
+  s.psum = s.esum + kFront;
+  s.bsum = s.psum + kFront;
+  s.pv = (float*)(s.bsum + kPBuckets);
+  s.bcnt = (int*)(s.pv + (size_t)kFront * front_seg(V));
+  s.pmax = (float*)(s.bcnt + kPBuckets);
   s.pcnt = (int*)(s.pmax + kFront);
   s.hist = s.pcnt + kFront;
   return s;
@@ -97,8 +124,15 @@ struct StepIO {
 constexpr int kCandLds = 512;      // candidates kept in LDS when they fit
 constexpr int kListsPerWave = kFront / (kThreads / 64);
 
+constexpr int kSortMax = 4096;  // entries sorted in LDS by the draw without top-k
+
 struct Smem {
-  unsigned radix[16 * kThreads];  // sort_large: per-thread digit counts, then offsets
+  union {
+    unsigned radix[16 * kThreads];  // sort_large: per-thread digit counts, then offsets
+    uint64_t keys[kSortMax];        // draw_parallel: (~probability bits, id), ascending
+  };
+  double dscan[kThreads / 64];
+  double dwork[4];
   Cand stage[kStage];
   Cand cand[kCandLds];
   Cand sel[kPartial];
@@ -160,7 +194,7 @@ __device__ __forceinline__ float min_p_threshold(float max_logit, float min_p) {
   return -1e30f;
 }
 
-__device__ __forceinline__ int effective_k(int top_k) {
+__host__ __device__ __forceinline__ int effective_k(int top_k) {
   return (top_k > 0 && top_k <= 256) ? top_k : 0;  // src/model.c:168-170
 }
 
@@ -595,6 +629,322 @@ __device__ void embed_next(int token, const StepIO& io) {
   for (int i = threadIdx.x; i < io.dm; i += kThreads) io.x[i] = row[i];
 }
 
+// ---------------------------------------------------------------------------
+// The draw without top-k (src/model.c:278-361) from sums in any order.
+//
+// The reference adds probabilities one by one in double, and only decisions
+// and fp32 roundings of those sums reach its result.  A double sum of n
+// non-negative terms is within (n - 1) 2^-53 of the exact one, relative,
+// whatever the order; so where a sum of the same terms in another order, widened
+// by twice that and more (sum_slack), decides or rounds the same way at both
+// ends, the reference's does too.  Where it does not (about once in 10^3
+// draws, from the fp32 roundings), or where the drawn token's probability is
+// tied in the min-heap's order, draw_parallel returns false and the
+// sequential code below runs.  So does it where more than kSortMax entries
+// share the bucket that decides, and for a top_k that cuts (above 256).
+// V = 50257, logits of spread 4 at temp = 0.8, top_p = 0.9: 2759 us per call
+// in turn on one thread (the sum, then the heap), 53.6 us this way.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ double wave_sum_f64(double v) {  // the same bits in every lane
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+// every thread has the same v: make the branches on it uniform (barriers
+// follow on both sides of them)
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+__device__ __forceinline__ double sum_slack(double sum, int n) { return sum * (double)n * 0x1p-51; }
+
+// (float)sum of the reference's sum, if every sum within the slack rounds alike
+__device__ __forceinline__ bool sure_float(double sum, int n, float* f) {
+  const double d = sum_slack(sum, n);
+  *f = (float)(sum - d);
+  return uni(*f == (float)(sum + d) && *f > 0.0f && *f < __builtin_inff());
+}
+
+// 1 / (float)sum (src/model.c:298)
+__device__ __forceinline__ bool softmax_scale(double sum, int n, float* inv) {
+  float f;
+  const bool ok = n > 0 && sure_float(sum, n, &f);
+  *inv = ok ? cr_divf(1.0f, f) : 0.0f;
+  return ok;
+}
+
+// block-wide inclusive prefix sum; *before = the sum in front of the thread
+__device__ double block_scan_f64(double v, double* before, Smem& sm) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double incl = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double u = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += u;
+  }
+  __syncthreads();
+  if (lane == 63) sm.dscan[wave] = incl;
+  __syncthreads();
+  double off = 0.0;
+  for (int w = 0; w < wave; ++w) off += sm.dscan[w];
+  const double up = __shfl_up(incl, 1, 64);
+  *before = lane ? off + up : off;
+  return off + incl;
+}
+
+// the listed probabilities of buckets lo..hi (at most kSortMax), as sorted
+// keys in sm.keys; returns their count
+__device__ int sort_buckets(const Scratch& sc, const int (&pc)[kListsPerWave], int seg, int lo,
+                            int hi, Smem& sm) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t below = (1ull << lane) - 1ull;
+  __syncthreads();
+  if (threadIdx.x == 0) sm.iwork[6] = 0;
+  __syncthreads();
+  constexpr int U = 4;  // 16-byte loads in flight per list
+#pragma unroll
+  for (int j = 0; j < kListsPerWave; ++j) {
+    const size_t base = (size_t)(wave * kListsPerWave + j) * seg;
+    for (int i0 = 0; i0 < pc[j]; i0 += 256 * U) {
+      float4 q[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)  // a list has room for seg entries, a multiple of 4
+        q[u] = *(const float4*)(sc.pv + base + min(i0 + 256 * u + 4 * lane, seg - 4));
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float v[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = i0 + 256 * u + 4 * lane + e;
+          const int b = p_bucket(v[e]);
+          const bool h = i < pc[j] && b >= lo && b <= hi;
+          const uint64_t m = __ballot(h);
+          if (!m) continue;
+          int at = 0;
+          if (lane == 0) at = atomicAdd(&sm.iwork[6], __popcll(m));
+          at = __builtin_amdgcn_readfirstlane(at) + __popcll(m & below);
+          if (h && at < kSortMax)
+            sm.keys[at] = (uint64_t)~__float_as_uint(v[e]) << 32 | (uint32_t)sc.pre[base + i].id;
+        }
+      }
+    }
+  }
+  __syncthreads();
+  const int n = min(uni(sm.iwork[6]), kSortMax);
+  int size = 64;
+  while (size < n) size *= 2;
+  for (int i = n + threadIdx.x; i < size; i += kThreads) sm.keys[i] = ~0ull;
+  // bitonic: larger probabilities first, equal ones by ascending id
+  for (int k = 2; k <= size; k *= 2)
+    for (int d = k / 2; d >= 1; d /= 2) {
+      __syncthreads();
+      for (int t = threadIdx.x; t < size / 2; t += kThreads) {
+        const int i = 2 * t - (t & (d - 1)), l = i + d;
+        const uint64_t a = sm.keys[i], b = sm.keys[l];
+        if ((a > b) == ((i & k) == 0)) {
+          sm.keys[i] = b;
+          sm.keys[l] = a;
+        }
+      }
+    }
+  __syncthreads();
+  return n;
+}
+
+__device__ __forceinline__ float key_prob(uint64_t k) { return __uint_as_float(~(uint32_t)(k >> 32)); }
+
+// first sorted entry whose running sum (from `base`) passes x -- is >= x
+// (INCL) or > x -- and whether that is sure; the running sum there in *at.
+// first: nothing comes before entry 0.  n if none passes.
+template <bool INCL>
+__device__ int find_key(int n, double base, double x, double slack, bool first, bool* sure,
+                        double* at, Smem& sm) {
+  double v[kSortMax / kThreads], own = 0.0, before;
+  const int i0 = threadIdx.x * (kSortMax / kThreads);
+#pragma unroll
+  for (int e = 0; e < kSortMax / kThreads; ++e) {
+    v[e] = i0 + e < n ? (double)key_prob(sm.keys[i0 + e]) : 0.0;
+    own += v[e];
+  }
+  block_scan_f64(own, &before, sm);
+  if (threadIdx.x == 0) sm.iwork[7] = n;
+  __syncthreads();
+  double run = base + before;
+  bool found = false;
+#pragma unroll
+  for (int e = 0; e < kSortMax / kThreads; ++e) {
+    run += v[e];
+    if (!found && i0 + e < n && (INCL ? run >= x : run > x)) {
+      found = true;
+      atomicMin(&sm.iwork[7], i0 + e);
+    }
+  }
+  __syncthreads();
+  const int j = uni(sm.iwork[7]);
+  if (j < n && j >= i0 && j < i0 + kSortMax / kThreads) {
+    double r = base + before;
+#pragma unroll
+    for (int e = 0; e < kSortMax / kThreads; ++e)
+      if (i0 + e <= j) {
+        sm.dwork[1] = r;
+        r += v[e];
+      }
+    sm.dwork[0] = r;
+  }
+  __syncthreads();
+  *at = sm.dwork[0];
+  *sure = uni(j < n && sm.dwork[0] > x + slack && ((first && j == 0) || sm.dwork[1] < x - slack));
+  __syncthreads();
+  return j;
+}
+
+// first bucket, from the largest probabilities down, whose running sum
+// passes x; in front of it: *sum and *cnt.  -1 if none passes.
+template <bool INCL>
+__device__ int find_bucket(const double (&s)[2], const int (&c)[2], double x, double* sum, int* cnt,
+                           Smem& sm) {
+  double sb;
+  block_scan_f64(s[0] + s[1], &sb, sm);
+  unsigned total;
+  const int cb = (int)block_scan((unsigned)(c[0] + c[1]), sm, &total);
+  if (threadIdx.x == 0) sm.iwork[7] = kPBuckets;
+  __syncthreads();
+  const double r0 = sb + s[0], r1 = r0 + s[1];
+  const int d = 2 * threadIdx.x;
+  if (c[0] && (INCL ? r0 >= x : r0 > x))
+    atomicMin(&sm.iwork[7], d);
+  else if (c[1] && (INCL ? r1 >= x : r1 > x))
+    atomicMin(&sm.iwork[7], d + 1);
+  __syncthreads();
+  const int at = uni(sm.iwork[7]);
+  if (at == d || at == d + 1) {
+    sm.dwork[2] = at == d ? sb : r0;
+    sm.iwork[5] = at == d ? cb : cb + c[0];
+  }
+  __syncthreads();
+  *sum = sm.dwork[2];
+  *cnt = uni(sm.iwork[5]);
+  __syncthreads();
+  return at == kPBuckets ? -1 : kPBuckets - 1 - at;
+}
+
+__device__ bool draw_parallel(const Scratch& sc, const int (&pc)[kListsPerWave], int seg,
+                              const SampleParams& p, uint64_t& rng, int* token, Smem& sm) {
+  static_assert(kFront == 64 && kPBuckets == 2 * kThreads, "lane / thread per list / buckets");
+  const int lane = threadIdx.x & 63;
+  const int mine = sc.pcnt[lane];
+  const int n = wave_sum_i32(mine);
+  float inv, f;
+  if (!softmax_scale(wave_sum_f64(sc.esum[lane]), n, &inv)) return false;
+  const double ps = sc.psum[lane], total = wave_sum_f64(ps);
+  const double slack = sum_slack(total, n);
+  uint64_t g = rng;
+  if (p.top_p >= 1.0f && (p.top_k <= 0 || p.top_k >= n)) {
+    // in index order: the list, then the entry the walk ends at
+    if (!sure_float(total, n, &f)) return false;
+    const double r = (double)__fmul_rn(rng_float(g), f);
+    double incl = ps;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double u = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += u;
+    }
+    const uint64_t hit = __ballot(mine > 0 && incl > r);
+    if (!hit) return false;
+    const int l = __ffsll((unsigned long long)hit) - 1;
+    const double base = l ? __shfl(incl, l - 1, 64) : 0.0;
+    const int cnt = __shfl(mine, l, 64);
+    const size_t at = (size_t)l * seg;
+    static_assert(kMaxVocab / kFront + 4 <= 4 * kThreads, "a list fits one pass");
+    double v[4], own = 0.0, before;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = 4 * threadIdx.x + e;
+      v[e] = i < cnt ? (double)sc.pv[at + i] : 0.0;
+      own += v[e];
+    }
+    block_scan_f64(own, &before, sm);
+    if (threadIdx.x == 0) sm.iwork[7] = -1;
+    __syncthreads();
+    double run = base + before;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = 4 * threadIdx.x + e;
+      const double next = run + v[e];
+      if (next > r + slack && (run < r - slack || (l == 0 && i == 0)))  // one entry at most
+        sm.iwork[7] = sc.pre[at + min(i, seg - 1)].id;
+      run = next;
+    }
+    __syncthreads();
+    *token = uni(sm.iwork[7]);
+    __syncthreads();
+    if (*token < 0) return false;
+    rng = g;
+    return true;
+  }
+  if (p.top_p >= 1.0f) return false;  // top_k > 256 alone: by the sort
+
+  // sorted: the cut at top_p
+  double s[2];
+  int c[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const int b = kPBuckets - 1 - 2 * (int)threadIdx.x - e;
+    s[e] = sc.bsum[b];
+    c[e] = sc.bcnt[b];
+  }
+  const double tp = (double)p.top_p;
+  double front = 0.0, kept = total;
+  int fcnt = 0, ncut = n, held = -1, n_held = 0;  // held: the bucket(s) in sm.keys
+  bool all = false, sure;
+  const int bc = find_bucket<true>(s, c, tp, &front, &fcnt, sm);
+  auto count_of = [&](int b) {  // the bucket's count, to every thread
+    const int t = (kPBuckets - 1 - b) / 2, e = (kPBuckets - 1 - b) & 1;
+    if ((int)threadIdx.x == t) sm.iwork[6] = e ? c[1] : c[0];
+    __syncthreads();
+    const int r = uni(sm.iwork[6]);
+    __syncthreads();
+    return r;
+  };
+  if (bc < 0) {
+    if (uni(total + slack >= tp)) return false;
+  } else {
+    const int cnt = count_of(bc);
+    all = fcnt + cnt <= kSortMax;
+    if (!all && cnt > kSortMax) return false;
+    if (all) front = 0.0, fcnt = 0;
+    n_held = sort_buckets(sc, pc, seg, bc, all ? kPBuckets - 1 : bc, sm);
+    held = bc;
+    const int j = find_key<true>(n_held, front, tp, slack, fcnt == 0, &sure, &kept, sm);
+    if (!sure) return false;
+    ncut = fcnt + j + 1;
+  }
+  if (p.top_k > 0 && p.top_k < ncut) return false;
+  if (!sure_float(kept, n, &f)) return false;
+  const double r = (double)__fmul_rn(rng_float(g), f);
+  if (!all) {
+    const int br = find_bucket<false>(s, c, r, &front, &fcnt, sm);
+    if (br < 0) return false;
+    if (br != held) {
+      if (count_of(br) > kSortMax) return false;
+      n_held = sort_buckets(sc, pc, seg, br, br, sm);
+    }
+  }
+  const int j = find_key<false>(n_held, front, r, slack, fcnt == 0, &sure, &kept, sm);
+  if (!sure || fcnt + j >= ncut) return false;
+  const uint64_t key = sm.keys[j];
+  // up to kPartial entries come out of the min-heap, whose order decides
+  // among equal ones; a full sort keeps them by index
+  if (n > kPartial && ncut <= kPartial) {
+    const uint32_t hi = (uint32_t)(key >> 32);
+    if (uni((j > 0 && (uint32_t)(sm.keys[j - 1] >> 32) == hi) ||
+            (j + 1 < n_held && (uint32_t)(sm.keys[j + 1] >> 32) == hi)))
+      return false;
+  }
+  *token = uni((int)(uint32_t)key);
+  rng = g;
+  return true;
+}
+
 }  // namespace
 
 // Front pass 1: logits[i] *= 1/temp over the block's segment and the
@@ -643,7 +993,8 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_scale(float* __restrict_
 }
 
 // Front pass 2, kFront blocks: with the global max (of the npart partial
-// maxima in pmax), each block adds its segment's counts to the 128-bucket
+// maxima in pmax), each block -- without top-k: also exp(logit - max) of its
+// candidates into pv and their sum; with top-k: -- adds its segment's counts to the 128-bucket
 // histogram over logits >= the min_p threshold (src/model.c:180-194) and
 // writes its pre-candidates: (i, logits[i]) with logits[i] >= the lowest
 // extraction threshold, in index order, to pre[block * seg ..].
@@ -669,9 +1020,18 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __rest
   const float pre_thresh =
       use_hist ? extract_threshold(max_logit, min_p_thresh, kBuckets - 1) : min_p_thresh;
   if (threadIdx.x < kBuckets) bhist[threadIdx.x] = 0;
+  __shared__ double wsum[NW];
+  // k_samp_probs adds to the buckets after this kernel
+  constexpr int kClear = kPBuckets / kFront;
+  if (!use_hist && threadIdx.x < kClear) {
+    sc.bsum[blockIdx.x * kClear + threadIdx.x] = 0.0;
+    sc.bcnt[blockIdx.x * kClear + threadIdx.x] = 0;
+  }
   __syncthreads();
   const uint64_t below = (1ull << lane) - 1ull;
   Cand* pre = sc.pre + (size_t)blockIdx.x * seg;
+  float* pv = sc.pv + (size_t)blockIdx.x * seg;
+  double esum = 0.0;
   int last = 0, off = 0;
   // the segment in rows of 4 * kFrontThreads entries (one row up to 65536
   // vocabulary entries), each compacted in index order after the last
@@ -717,8 +1077,21 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __rest
     for (int e = 0; e < 4; ++e) pos += __popcll(m[e] & below);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (h[e]) pre[pos++] = Cand{i + e, v[e]};
+      if (h[e]) {
+        if (!use_hist) {  // the softmax numerator (src/model.c:292-297)
+          const float ex = libm::expf_glibc(__fsub_rn(v[e], max_logit));
+          pv[pos] = ex;
+          esum += (double)ex;
+        }
+        pre[pos++] = Cand{i + e, v[e]};
+      }
     off += row;
+  }
+  if (!use_hist) {
+    esum = wave_sum_f64(esum);
+    if (lane == 0) wsum[wave] = esum;
+    __syncthreads();
+    if (threadIdx.x == 0) sc.esum[blockIdx.x] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
   }
   if (use_hist) {
     last = wave_sum_i32(last);
@@ -730,7 +1103,47 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __rest
   if (threadIdx.x == 0) sc.pcnt[blockIdx.x] = off;
 }
 
-// The rest of sample_advanced on one 1024-thread block, after the two front
+// Front pass 3 (no top-k), kFront blocks: the probabilities pv * 1/sum, their
+// sum per block, and the count and sum of each value bucket over all blocks.
+__global__ __launch_bounds__(kFrontThreads) void k_samp_probs(int V, void* scratch,
+                                                              const int* ctl) {
+  __shared__ double bsum[kPBuckets];
+  __shared__ int bcnt[kPBuckets];
+  __shared__ double wsum[kFrontThreads / 64];
+  if (step_stopped(ctl)) return;
+  const Scratch sc = scratch_of(scratch, V);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cnt = sc.pcnt[blockIdx.x];
+  const int n = wave_sum_i32(sc.pcnt[lane]);
+  for (int b = threadIdx.x; b < kPBuckets; b += kFrontThreads) {
+    bsum[b] = 0.0;
+    bcnt[b] = 0;
+  }
+  float inv;
+  const bool ok = softmax_scale(wave_sum_f64(sc.esum[lane]), n, &inv);
+  __syncthreads();
+  if (!ok) return;  // k_sample finds the same and takes the sequential path
+  float* pv = sc.pv + (size_t)blockIdx.x * front_seg(V);
+  double sum = 0.0;
+  for (int i = threadIdx.x; i < cnt; i += kFrontThreads) {
+    const float v = __fmul_rn(pv[i], inv);
+    pv[i] = v;
+    sum += (double)v;
+    const int b = p_bucket(v);
+    atomicAdd(&bcnt[b], 1);
+    unsafeAtomicAdd(&bsum[b], (double)v);
+  }
+  sum = wave_sum_f64(sum);
+  if (lane == 0) wsum[wave] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) sc.psum[blockIdx.x] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+  for (int b = threadIdx.x; b < kPBuckets; b += kFrontThreads)
+    if (bcnt[b]) {
+      atomicAdd(&sc.bcnt[b], bcnt[b]);
+      unsafeAtomicAdd(&sc.bsum[b], bsum[b]);
+    }
+}
+
+// The rest of sample_advanced on one 1024-thread block, after the front
 // passes: the cutoff bucket, the candidates filtered from the pre-candidate
 // lists in order, selection, softmax, sorting and the draw; then the step
 // bookkeeping and the next token's embedding (StepIO).  Leaves the
@@ -820,7 +1233,7 @@ __global__ __launch_bounds__(1024) void k_sample(const float* __restrict__ logit
       }
       token = filter_and_sample(src, n, p.top_p, 0, rng, sm);
     }
-  } else {
+  } else if (!draw_parallel(sc, pc, seg, p, rng, &token, sm)) {
     // no top-k: every candidate over the min_p threshold (src/model.c:278-300)
     int n = gather(sc, pc, seg, min_p_thresh, sc.probs, &probs, sm);
     if (n == 0) {
@@ -904,8 +1317,10 @@ __global__ __launch_bounds__(1024) void k_sample_greedy(const float* __restrict_
 
 size_t sample_scratch_bytes(int V) {
   if (V < 1) return 0;
-  return ((size_t)V + (size_t)kFront * front_seg(V)) * sizeof(Cand) +
-         (2 * kFront + kBuckets) * sizeof(int);
+  const size_t lists = (size_t)kFront * front_seg(V);
+  // + 32: the two alignments of scratch_of
+  return ((size_t)V + lists) * sizeof(Cand) + (2 * kFront + kPBuckets) * sizeof(double) +
+         (lists + kPBuckets + 2 * kFront + kBuckets) * sizeof(int) + 32;
 }
 
 // pmax/npart: the maxima of logits already scaled by 1/temp (the LM head's
@@ -932,6 +1347,9 @@ hipError_t launch_sample(float* logits, int V, float temp, float min_p, float to
   }
   hipLaunchKernelGGL(k_samp_hist, dim3(kFront), dim3(kFrontThreads), 0, s, logits, V, p, scratch,
                      pmax, npart, gated ? (const int*)ctl : nullptr);
+  if (effective_k(top_k) == 0)
+    hipLaunchKernelGGL(k_samp_probs, dim3(kFront), dim3(kFrontThreads), 0, s, V, scratch,
+                       gated ? (const int*)ctl : nullptr);
   hipLaunchKernelGGL(k_sample, dim3(1), dim3(kThreads), 0, s, logits, V, p, rng_state, scratch,
                      pmax, npart, io);
   return hipGetLastError();
