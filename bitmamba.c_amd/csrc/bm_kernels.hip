@@ -135,6 +135,177 @@ __global__ __launch_bounds__(QT) void k_quantize(const float* __restrict__ x, in
 }
 
 // ---------------------------------------------------------------------------
+// Quantizer of one token per 256-thread block for n <= 256 E: the token stays
+// in registers, wave j runs chain j of the sum of squares (chain_wave,
+// bm_dev.h).  VEC: 16-byte loads (n, the row stride and the pointers multiples
+// of 4 floats); otherwise thread t owns columns t + 256 i.
+//
+// Latency decides where the tokens leave the chip idle: launch, the round trip
+// for x, the chains, and the LDS passes.  n = 8192: 24.9 -> 6.6 us at 2 tokens,
+// 203 -> 45.6 us at 4096 against k_quantize (one lane per chain, x read three
+// times); n = 2048 and 4096 at launch_quantize.
+// ---------------------------------------------------------------------------
+template <int E, bool VEC>
+__global__ __launch_bounds__(QT) void k_quantize_tok(
+    const float* __restrict__ x, int n, int x_stride, const float* __restrict__ gamma,
+    float* __restrict__ x_norm, int8_t* __restrict__ xq, int quant_stride,
+    float* __restrict__ scale_out, float* __restrict__ max_out, uint8_t* __restrict__ act,
+    size_t act_stride, bool nib) {
+  constexpr int S = chain_floats(E), PAD = chain_pad(E);
+  __shared__ __attribute__((aligned(16))) float sq[4 * S];
+  __shared__ __attribute__((aligned(16))) int8_t q8[QT * E];
+  __shared__ float s_sum[4], s_max[4];
+  const int m = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const float* __restrict__ xr = x + (size_t)m * x_stride;
+  const int n4 = n & ~3;
+
+  // value i of the thread: column col(i); loads unconditional from clamped
+  // columns, zeros past n
+  auto col = [&](int i) { return VEC ? 4 * (tid + QT * (i >> 2)) + (i & 3) : tid + QT * i; };
+  float v[E], g[E];
+  if constexpr (VEC) {
+#pragma unroll
+    for (int i = 0; i < E; i += 4) {
+      const int c = min(col(i), n - 4);
+      const float4 a = *(const float4*)(xr + c), b = *(const float4*)(gamma + c);
+      v[i] = a.x, v[i + 1] = a.y, v[i + 2] = a.z, v[i + 3] = a.w;
+      g[i] = b.x, g[i + 1] = b.y, g[i + 2] = b.z, g[i + 3] = b.w;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      const int c = min(col(i), n - 1);
+      v[i] = xr[c];
+      g[i] = gamma[c];
+    }
+  }
+  float tail[3];  // the squares after the chains (src/kernel.c:88), the same in every thread
+#pragma unroll
+  for (int k = 0; k < 3; ++k) tail[k] = xr[min(n4 + k, n - 1)];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const int c = col(i), e = c >> 2;
+    const float t = c < n4 ? v[i] : 0.0f;
+    sq[(c & 3) * S + e + PAD * (e / E)] = __fmul_rn(t, t);
+  }
+  __syncthreads();
+  const float cs = chain_wave_lds<E>(sq + wave * S, 0.0f);
+  if (lane == 0) s_sum[wave] = cs;
+  __syncthreads();
+  float sum = __fadd_rn(__fadd_rn(__fadd_rn(s_sum[0], s_sum[1]), s_sum[2]), s_sum[3]);
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    if (n4 + k < n) sum = __fadd_rn(sum, __fmul_rn(tail[k], tail[k]));
+  const float rms = cr_divf(1.0f, cr_sqrtf(__fadd_rn(cr_divf(sum, (float)n), 1e-6f)));
+
+  float mx = 0.0f;
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    v[i] = __fmul_rn(__fmul_rn(v[i], rms), g[i]);
+    if (col(i) < n) mx = fmaxf(mx, fabsf(v[i]));
+  }
+  mx = wave_max_f32(mx);
+  if (lane == 0) s_max[wave] = mx;
+  __syncthreads();
+  const float max_abs = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
+  const float scale_x = cr_divf(127.0f, __fadd_rn(max_abs, 1e-5f));
+  if (tid == 0) {
+    if (scale_out) scale_out[m] = scale_x;
+    if (max_out) max_out[m] = max_abs;
+  }
+  int q[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const float t = __fmul_rn(v[i], scale_x);
+    const int r = (int)__fadd_rn(t, t >= 0.0f ? 0.5f : -0.5f);
+    q[i] = col(i) < n ? (r > 127 ? 127 : (r < -128 ? -128 : r)) : 0;
+  }
+  if constexpr (VEC) {
+#pragma unroll
+    for (int i = 0; i < E; i += 4) {
+      const int c = col(i);
+      *(uint32_t*)(q8 + c) = (uint32_t)(q[i] & 255) | (uint32_t)(q[i + 1] & 255) << 8 |
+                             (uint32_t)(q[i + 2] & 255) << 16 | (uint32_t)(q[i + 3] & 255) << 24;
+      if (x_norm && c < n)
+        *(float4*)(x_norm + (size_t)m * n + c) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      const int c = col(i);
+      q8[c] = (int8_t)q[i];
+      if (x_norm && c < n) x_norm[(size_t)m * n + c] = v[i];
+    }
+  }
+  if (!xq && !act) return;
+  __syncthreads();
+  // 16 columns per thread: the caller's int8 row, the activation workspace
+  const int n_groups = (n + 15) >> 4;
+  int8_t* __restrict__ qrow = xq ? xq + (size_t)m * quant_stride : nullptr;
+  uint8_t* __restrict__ arow = act ? act + (size_t)m * act_stride : nullptr;
+  const bool vec_q = ((uintptr_t)qrow & 15) == 0;
+#pragma unroll
+  for (int g0 = 0; g0 < 16 * E; g0 += QT) {
+    const int gr = g0 + tid;
+    uint4 raw = make_uint4(0, 0, 0, 0);
+    if (gr < n_groups) raw = *(const uint4*)(q8 + 16 * gr);
+    const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+    int b[16], qsum = 0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      b[j] = (int)(int8_t)(w[j >> 2] >> (8 * (j & 3)));
+      qsum += b[j];
+    }
+    if (qrow && gr < n_groups) {
+      if (vec_q && 16 * gr + 16 <= n) {
+        *(uint4*)(qrow + 16 * gr) = raw;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+          if (16 * gr + j < n) qrow[16 * gr + j] = (int8_t)b[j];
+      }
+    }
+    if (arow) {
+      if (gr < n_groups) write_act_group(arow, n, gr, b, nib);
+      // 64 groups = one 1024-column slice = one wave of this pass
+      const int ssum = wave_sum_i32(qsum);
+      const int slice = (g0 >> 6) + wave;
+      if (lane == 0 && slice < slices_of(n)) ((int*)arow)[slice] = ssum;
+    }
+  }
+}
+
+template <int E>
+static void quantize_tok_t(const float* x, int M, int n, int x_stride, const float* gamma,
+                           float* x_norm, int8_t* xq, int quant_stride, float* scale_x,
+                           float* max_out, uint8_t* act, bool nibbles, hipStream_t s) {
+  const bool vec = n % 4 == 0 && x_stride % 4 == 0 && (uintptr_t)x % 16 == 0 &&
+                   (uintptr_t)gamma % 16 == 0 && (!x_norm || (uintptr_t)x_norm % 16 == 0);
+  if (vec)
+    hipLaunchKernelGGL((k_quantize_tok<E, true>), dim3(M), dim3(QT), 0, s, x, n, x_stride, gamma,
+                       x_norm, xq, quant_stride, scale_x, max_out, act, act_row_bytes(n), nibbles);
+  else
+    hipLaunchKernelGGL((k_quantize_tok<E, false>), dim3(M), dim3(QT), 0, s, x, n, x_stride, gamma,
+                       x_norm, xq, quant_stride, scale_x, max_out, act, act_row_bytes(n), nibbles);
+}
+
+// false beyond n = 8192
+static bool quantize_tok(const float* x, int M, int n, int x_stride, const float* gamma,
+                         float* x_norm, int8_t* xq, int quant_stride, float* scale_x,
+                         float* max_out, uint8_t* act, bool nibbles, hipStream_t s) {
+  if (n < 1 || n > 8192) return false;
+  auto go = [&](auto e) {
+    quantize_tok_t<decltype(e)::value>(x, M, n, x_stride, gamma, x_norm, xq, quant_stride, scale_x,
+                                       max_out, act, nibbles, s);
+  };
+  if (n <= 1024) go(std::integral_constant<int, 4>());
+  else if (n <= 2048) go(std::integral_constant<int, 8>());
+  else if (n <= 4096) go(std::integral_constant<int, 16>());
+  else go(std::integral_constant<int, 32>());
+  return true;
+}
+
+// ---------------------------------------------------------------------------
 // Quantizer for n = 1024 * G (G in {1, 2, 4}): one wave per token, four
 // tokens per block (two at G = 4), no block barriers.  Lane l keeps the 16-column groups
 // l + 64i in registers; the squares pass through the wave's own LDS region
@@ -1424,7 +1595,19 @@ hipError_t launch_quantize(const float* x, int M, int n, int x_stride, const flo
   // one wave per token when the rows allow 16-byte loads of whole groups
   const bool aligned = ((uintptr_t)x % 16 == 0) && (x_stride % 4 == 0) &&
                        ((uintptr_t)gamma % 16 == 0) && (!x_norm || (uintptr_t)x_norm % 16 == 0);
-  if (aligned && (n == 1024 || n == 2048 || n == 4096)) {
+  const bool wave = aligned && (n == 1024 || n == 2048 || n == 4096);
+  // a block per token up to where the per-wave kernel's better use of the
+  // issue slots wins (us per call, wave / block: n = 2048 5.19 / 4.46 at 13
+  // tokens, 5.93 / 5.08 at 512, 6.14 / 6.17 at 768, 8.17 / 10.67 at 2048;
+  // n = 4096 7.51 / 5.12, 8.53 / 6.71, 11.07 / 9.54 at 1024, 14.66 / 15.22 at
+  // 2048; n = 1024 4.28 / 4.23 at 13, 4.21 / 4.70 at 512); fast mode sums as
+  // a tree in the per-wave kernel
+  const int block_max = n == 2048 ? 640 : (n == 4096 ? 1536 : 0);
+  if ((!wave || (!fast && M <= block_max)) &&
+      quantize_tok(x, M, n, x_stride, gamma, x_norm, xq, quant_stride, scale_x, nullptr, act,
+                   nibbles, s))
+    return hipGetLastError();
+  if (wave) {
     const int tpb = quantize_wave_tpb(n);
     const dim3 grid((M + tpb - 1) / tpb), block(64 * tpb);
     const size_t lds = quantize_wave_lds(n);
@@ -1454,6 +1637,8 @@ hipError_t launch_residual_add(float* x, const float* o, size_t n, hipStream_t s
 
 hipError_t launch_rms_norm(const float* x, int n, const float* gamma, float* out, float* max_out,
                            hipStream_t s) {
+  if (quantize_tok(x, 1, n, n, gamma, out, nullptr, 0, nullptr, max_out, nullptr, false, s))
+    return hipGetLastError();
   hipLaunchKernelGGL(k_quantize, dim3(1), dim3(QT), 0, s, x, n, n, gamma, out, (int8_t*)nullptr,
                      0, (float*)nullptr, max_out, (uint8_t*)nullptr, (size_t)0);
   return hipGetLastError();

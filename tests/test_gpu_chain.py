@@ -58,3 +58,31 @@ def test_one_token_prologue(hip, K):
         same_bits(ds.download(1, np.float32), osc, "scale row %d" % i)
         ref, _, _ = native.orc_bitlinear(x[i:i + 1], packed, N, K, 0.02, g)
         same_bits(do.download(N, np.float32), ref[0], "out row %d" % i)
+
+
+@pytest.mark.parametrize("n", [1, 3, 5, 1000, 1024, 1027, 2048, 2052, 4096, 4099, 8190, 8192, 8200])
+def test_token_block_quantizer(hip, n):
+    """The per-token quantizer at few tokens: 16-byte and scalar loads, every
+    elements-per-lane class, the K % 4 tail, int8 rows of any stride."""
+    x = rows_for(n, 9 * n) if n >= 16 else rnd_rows(n)
+    M = x.shape[0]
+    g = (np.random.default_rng(n).standard_normal(n) * 0.02).astype(np.float32)
+    on, oq, osc, _ = native.orc_quantize_rows(x, g)
+    for stride, qs in ((n, n), (n + 1, n + 3), ((n + 3) // 4 * 4, (n + 15) // 16 * 16)):
+        print("quantize n=%d x stride=%d int8 stride=%d" % (n, stride, qs), flush=True)
+        xs = np.zeros((M, stride), np.float32)
+        xs[:, :n] = x
+        dx, dg, dn, ds = DB.from_array(xs), DB.from_array(g), DB(4 * M * n), DB(4 * M)
+        dq = DB.from_array(np.full((M, qs), 99, np.int8))
+        bh.check(hip.bm_hip_quantize_dev(dx.ptr, M, n, stride, dg.ptr, dn.ptr, dq.ptr, qs, ds.ptr,
+                                         None, None), "quantize")
+        hip.bm_hip_synchronize()
+        same_bits(dn.download((M, n), np.float32), on, "x_norm")
+        q = dq.download((M, qs), np.int8)
+        np.testing.assert_array_equal(q[:, :n], oq)
+        assert (q[:, n:] == 99).all()
+        same_bits(ds.download(M, np.float32), osc, "scale")
+
+
+def rnd_rows(n):
+    return np.random.default_rng(n).standard_normal((5, n)).astype(np.float32)
