@@ -86,3 +86,34 @@ def test_token_block_quantizer(hip, n):
 
 def rnd_rows(n):
     return np.random.default_rng(n).standard_normal((5, n)).astype(np.float32)
+
+
+@pytest.mark.parametrize("M", [1, 2, 7, 8, 9, 37])
+@pytest.mark.parametrize("K", [1, 3, 4, 63, 1000, 1023, 1024 + 4, 1025, 2050, 4100])
+def test_generic_product(hip, M, K):
+    """Widths that are not multiples of 64: int32 totals and the fp32 epilogue
+    with its remainder columns; rows that do not fill a block; code 11."""
+    for N in (1, 15, 17, 130):
+        print("generic M=%d K=%d N=%d" % (M, K, N), flush=True)
+        r = np.random.default_rng(M * 131 + K * 7 + N)
+        kb = (K + 3) // 4
+        packed = r.integers(0, 256, (N, kb)).astype(np.uint8)
+        if K % 4:
+            packed[:, -1] &= (1 << (2 * (K % 4))) - 1
+        x = r.standard_normal((M, K)).astype(np.float32)
+        g = (r.standard_normal(K) * 0.02).astype(np.float32)
+        dx, dg, dw = DB.from_array(x), DB.from_array(g), DB.from_array(packed)
+        do, dq, ds = DB(4 * M * N), DB(M * K), DB(4 * M)
+        da = DB(hip.bm_hip_act_bytes(M, K))
+        bh.check(hip.bm_hip_bitlinear_dev(dx.ptr, M, K, dg.ptr, dw.ptr, N, 0.02, 0, do.ptr, dq.ptr,
+                                          K, ds.ptr, da.ptr, None), "bitlinear")
+        hip.bm_hip_synchronize()
+        ref, _, _ = native.orc_bitlinear(x, packed, N, K, 0.02, g)
+        same_bits(do.download((M, N), np.float32), ref, "out")
+        xq = r.integers(-128, 128, (M, K + 3)).astype(np.int8)
+        dxq, dt = DB.from_array(xq), DB(4 * M * N)
+        bh.check(hip.bm_hip_ternary_gemm_i32_dev(dxq.ptr, M, K + 3, dw.ptr, N, K, 0, dt.ptr, da.ptr,
+                                                 None), "int32")
+        hip.bm_hip_synchronize()
+        want = native.orc_gemm_i32(np.ascontiguousarray(xq[:, :K]), packed, N, K)
+        np.testing.assert_array_equal(dt.download((M, N), np.int32), want)
