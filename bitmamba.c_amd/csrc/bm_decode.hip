@@ -37,19 +37,6 @@ constexpr int kDoneArmed = 1, kDoneStopped = 2;
 __device__ __forceinline__ bool is_end_token(int t) { return t == 50256 || t == 0; }
 constexpr int kHist = 256;
 
-// the libm tables, in device memory or copied to LDS
-struct LibmTabs {
-  uint64_t exp2[32];
-  double invc[16], logc[16];
-};
-// the copy's word i (of 64), lane by lane
-__device__ __forceinline__ uint64_t libm_tab_word(int i) {
-  const uint64_t* src = i < 32   ? libm::kExp2Tab + i
-                        : i < 48 ? (const uint64_t*)libm::kLogInvC + (i - 32)
-                                 : (const uint64_t*)libm::kLogC + (i - 48);
-  return *src;
-}
-
 __device__ __forceinline__ float silu_r(float x, const uint64_t* exp2 = libm::kExp2Tab) {
   return cr_divf(x, __fadd_rn(1.0f, libm::expf_tab(-x, exp2)));
 }
@@ -1011,9 +998,9 @@ __global__ __launch_bounds__(256) void k_inproj_ssm(const float* __restrict__ x,
   const float dtb = a.dt_bias[h], Ah = a.A[h];
   // the tables of expf and logf, copied to LDS by wave 3: a lookup in device
   // memory costs a cache miss in every launch, and the decay has three in a row
-  __shared__ LibmTabs s_libm;
+  __shared__ libm::Tabs s_libm;
   uint64_t tab_word = 0;
-  if (wave == 3) tab_word = libm_tab_word(lane);
+  if (wave == 3) tab_word = libm::tab_word(lane);
 
   const Lds l = lds_carve(lds, WP ? 1024 * C : K);
   float scale_x;

@@ -131,5 +131,19 @@ BM_HD float logf_tab(float x, const double* invc_tab, const double* logc_tab) {
 }
 BM_HD float logf_glibc(float x) { return logf_tab(x, kLogInvC, kLogC); }
 
+#if defined(__HIPCC__)
+// the tables as a kernel copies them to LDS, 64 words, one per lane of a wave
+struct Tabs {
+  uint64_t exp2[32];
+  double invc[16], logc[16];
+};
+__device__ __forceinline__ uint64_t tab_word(int i) {
+  const uint64_t* src = i < 32   ? kExp2Tab + i
+                        : i < 48 ? (const uint64_t*)kLogInvC + (i - 32)
+                                 : (const uint64_t*)kLogC + (i - 48);
+  return *src;
+}
+#endif
+
 }  // namespace libm
 }  // namespace bm

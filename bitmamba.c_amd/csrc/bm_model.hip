@@ -33,18 +33,21 @@ enum { CTL_POS = 0, CTL_DONE = 1, CTL_STEP = 2, CTL_HCOUNT = 3, CTL_TOKEN = 4, C
 constexpr int kDoneArmed = 1, kDoneStopped = 2;
 constexpr int kHistory = 256;  // HISTORY_MAX (src/main.c:19)
 
-__device__ __forceinline__ float silu_ref(float x) {
+__device__ __forceinline__ float silu_ref(float x, const uint64_t* exp2 = libm::kExp2Tab) {
   // x / (1.0f + expf(-x))  (src/bitmamba.h:234-237)
-  return cr_divf(x, __fadd_rn(1.0f, libm::expf_glibc(-x)));
+  return cr_divf(x, __fadd_rn(1.0f, libm::expf_tab(-x, exp2)));
 }
 
-__device__ __forceinline__ float softplus_ref(float x) {
+__device__ __forceinline__ float softplus_ref(float x, const uint64_t* exp2 = libm::kExp2Tab,
+                                              const double* invc = libm::kLogInvC,
+                                              const double* logc = libm::kLogC) {
   // x > 20 ? x : logf(1.0f + expf(x))  (src/bitmamba.h:238-243)
   if (x > 20.0f) return x;
-  return libm::logf_glibc(__fadd_rn(1.0f, libm::expf_glibc(x)));
+  return libm::logf_tab(__fadd_rn(1.0f, libm::expf_tab(x, exp2)), invc, logc);
 }
 
-// Prefill SSM (ssm_batch_worker, src/block.c:127-160) in three phases.  Of
+// Prefill SSM (ssm_batch_worker, src/block.c:127-160) in three phases
+// (k_ssm_fused below runs them as one pipeline).  Of
 // scalar_ssm_inner's per-token work (src/kernel.c:34-70) only the state
 // update st = st * decay + xa * (B * dt) and y = (st * C + xa * D) * silu(z)
 // depend on the previous token; dt, decay, the depthwise conv over the
@@ -258,6 +261,199 @@ __global__ __launch_bounds__(256) void k_ssm_out(const float* __restrict__ pre,
                     silu_ref(proj[(size_t)(t0 + t) * pd + zoff]));
     }
   }
+}
+
+// The three phases in one kernel, for head dims that are multiples of 16: a
+// block owns 16 channels of one head for the whole prompt, and its waves are
+// stages of a pipeline over tiles of 64 tokens (iteration i): wave 1 forms
+// dt, decay and B * dt of tile i (lane = token), waves 2..9 the conv, silu and
+// products of tile i - 1, wave 0 runs the recurrence over tile i - 2 (lane =
+// channel, 16 lanes; raised wave priority), and waves 2..9 the outputs of tile
+// i - 3.  xa * B * dt and the states pass through LDS, xa * D stays in the
+// registers of the thread that needs it two iterations later, so of the
+// three-phase version's planes nothing goes through memory.  A tile's inputs
+// are loaded one iteration ahead; loads and stores are unconditional (through
+// bounds-checked buffers) so that a wait covers only what it needs.  Tokens past n carry decay 1 and xa * B * dt = -0.
+// Bound by instruction issue: the SIMDs that hold wave 0 and wave 1 beside two
+// task waves issue ~650 vector instructions per tile (silu ~55 each).  1B
+// shape, 1024 tokens, per layer: 23.7 us against 17.6 + 13.9 + 13.9 us for
+// the three kernels (the planes were ~130 MB of traffic); the prefill of 1024
+// tokens 2.515 -> 1.854 ms, of 8 tokens 0.917 -> 0.663 ms, with the
+// quantizers' change in both.  With plain loads whose row or ring address is
+// chosen per lane (a branch around each) 27.3 us.
+constexpr int kFc = 16, kFt = 64, kFtasks = 8;  // channels, tile, task waves
+
+__global__ __launch_bounds__(64 * (kFtasks + 2)) void k_ssm_fused(
+    const float* __restrict__ proj, int pd, int n, int di, int hd,
+    const float* __restrict__ dt_bias, const float* __restrict__ A, const float* __restrict__ cw,
+    const float* __restrict__ cb, float* __restrict__ cs, float* __restrict__ ssm,
+    const float* __restrict__ D, const int* __restrict__ ctl, float* __restrict__ y) {
+  constexpr int ROW = kFt + 4;  // 16 lanes' 16-byte accesses on different banks
+  __shared__ libm::Tabs tabs;
+  __shared__ __attribute__((aligned(16))) float s_bdt[4][kFt], s_dec[4][kFt], s_c[4][kFt];
+  __shared__ __attribute__((aligned(16))) float s_xb[2][kFc * ROW], s_st[2][kFc * ROW];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // neighbouring channel groups share cache lines: on one XCD (blocks are
+  // dealt to the 8 XCDs in turn)
+  const int nb = gridDim.x;
+  const int blk = nb % 8 == 0 ? (int)(blockIdx.x % 8) * (nb / 8) + (int)blockIdx.x / 8
+                              : (int)blockIdx.x;
+  const int h = blk * kFc / hd, c0 = blk * kFc;
+  const float* __restrict__ ph = proj + (size_t)h * (2 * hd + 3);  // z | x | B | C | dt
+  const int nt = (n + kFt - 1) / kFt;
+  const int pos0 = ctl[CTL_POS];
+  if (tid < 64) ((uint64_t*)&tabs)[tid] = libm::tab_word(tid);
+
+  if (wave == 0) {
+    __builtin_amdgcn_s_setprio(3);
+    const int c = lane & (kFc - 1), idx = c0 + c;
+    float st = ssm[idx];
+    __syncthreads();
+    for (int it = 0; it < nt + 3; ++it) {
+      const int k = it - 2;
+      if (k >= 0 && k < nt) {
+        const float* __restrict__ xb = s_xb[k & 1] + c * ROW;
+        const float* __restrict__ dec = s_dec[k & 3];
+        float* __restrict__ o = s_st[k & 1] + c * ROW;
+#pragma unroll
+        for (int q = 0; q < kFt; q += 4) {
+          const float4 x = *(const float4*)(xb + q), d = *(const float4*)(dec + q);
+          float4 r;
+          r.x = __fadd_rn(__fmul_rn(st, d.x), x.x);
+          r.y = __fadd_rn(__fmul_rn(r.x, d.y), x.y);
+          r.z = __fadd_rn(__fmul_rn(r.y, d.z), x.z);
+          st = r.w = __fadd_rn(__fmul_rn(r.z, d.w), x.w);
+          if (lane < kFc) *(float4*)(o + q) = r;
+        }
+      }
+      __syncthreads();
+    }
+    // every input has been read: the state, and the conv ring as the token
+    // loop leaves it (the inputs of the last three tokens)
+    if (lane < kFc) {
+      ssm[idx] = st;
+      for (int k = max(0, n - 3); k < n; ++k)
+        cs[(size_t)((pos0 + k) % 3) * di + idx] = ph[(size_t)k * pd + hd + (idx - h * hd)];
+    }
+  } else if (wave == 1) {
+    const float bias = dt_bias[h], Ah = A[h];
+    float vB, vC, vd;
+    auto fetch = [&](int tile) __attribute__((always_inline)) {
+      const float* __restrict__ p = ph + (size_t)min(tile * kFt + lane, n - 1) * pd + 2 * hd;
+      vB = p[0];
+      vC = p[1];
+      vd = p[2];
+    };
+    fetch(0);
+    __syncthreads();
+    for (int it = 0; it < nt + 3; ++it) {
+      const float B = vB, C = vC, d = vd;
+      fetch(it + 1);
+      if (it < nt) {
+        const float dt_val = softplus_ref(__fadd_rn(d, bias), tabs.exp2, tabs.invc, tabs.logc);
+        const float decay = libm::expf_tab(__fmul_rn(Ah, dt_val), tabs.exp2);
+        const bool in = it * kFt + lane < n;
+        s_bdt[it & 3][lane] = __fmul_rn(B, dt_val);
+        s_dec[it & 3][lane] = in ? decay : 1.0f;
+        s_c[it & 3][lane] = C;
+      }
+      __syncthreads();
+    }
+  } else {
+    // two tokens of one channel per lane and tile
+    const int c = lane & (kFc - 1), idx = c0 + c;
+    const int tw = 8 * (wave - 2) + 2 * (lane >> 4);  // token in the tile
+    const float* __restrict__ pz = ph + (idx - h * hd);
+    const float w0 = cw[idx], w1 = cw[di + idx], w2 = cw[2 * di + idx], w3 = cw[3 * di + idx];
+    const float bias = cb[idx], Dv = D[idx];
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(y, 0, (int)((unsigned)n * (unsigned)di * 4u),
+                                                  0x00027000);
+    // inputs of tokens t-3 .. t+1; rows outside the batch read as 0
+    auto rproj = __builtin_amdgcn_make_buffer_rsrc((void*)proj, 0,
+                                                   (int)((unsigned)n * (unsigned)pd * 4u), 0x00027000);
+    const unsigned row = (unsigned)pd * 4u;
+    const unsigned oz = (unsigned)((pz - proj) * 4) + (unsigned)tw * row;
+    const unsigned ox = oz + (unsigned)hd * 4u - 3u * row;  // before the batch: past any buffer
+    float xv[5], zv[2];
+    auto fetch_x = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+      for (int k = 0; k < 5; ++k)
+        xv[k] = __int_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(rproj, (int)(ox + (unsigned)(tile * kFt + k) * row), 0, 0));
+    };
+    auto fetch_z = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        zv[e] = __int_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(rproj, (int)(oz + (unsigned)(tile * kFt + e) * row), 0, 0));
+    };
+    // the three inputs before the prompt, x[t] at conv ring position pos0 + 3 + t
+    float ring[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) ring[k] = cs[(size_t)((pos0 + k) % 3) * di + idx];
+    float xad[3][2] = {};  // of tiles a, a - 1, a - 2
+    fetch_x(0);
+    fetch_z(0);
+    __syncthreads();
+    for (int it = 0; it < nt + 3; ++it) {
+      const int a = it - 1, o = it - 3;
+      float conv[2], z[2];
+      if (a == 0) {  // tile 0's first lanes reach back before the prompt
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          if (tw - 3 + k < 0) xv[k] = tw == 0 ? ring[k] : ring[2];
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        conv[e] = __fadd_rn(bias, __fmul_rn(xv[e], w0));
+        conv[e] = __fadd_rn(conv[e], __fmul_rn(xv[e + 1], w1));
+        conv[e] = __fadd_rn(conv[e], __fmul_rn(xv[e + 2], w2));
+        conv[e] = __fadd_rn(conv[e], __fmul_rn(xv[e + 3], w3));
+        z[e] = zv[e];
+      }
+      fetch_x(max(a + 1, 0));
+      fetch_z(max(o + 1, 0));
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        xad[2][e] = xad[1][e];
+        xad[1][e] = xad[0][e];
+      }
+      if (a >= 0 && a < nt) {
+        float xb[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float xa = silu_ref(conv[e], tabs.exp2);
+          xb[e] = a * kFt + tw + e < n ? __fmul_rn(xa, s_bdt[a & 3][tw + e]) : -0.0f;
+          xad[0][e] = __fmul_rn(xa, Dv);
+        }
+        *(float2*)(s_xb[a & 1] + c * ROW + tw) = make_float2(xb[0], xb[1]);
+      }
+      float out[2] = {0.0f, 0.0f};
+      if (o >= 0) {
+        const float2 s2 = *(const float2*)(s_st[o & 1] + c * ROW + tw);
+        const float sv[2] = {s2.x, s2.y};
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          out[e] = __fmul_rn(__fadd_rn(__fmul_rn(sv[e], s_c[o & 3][tw + e]), xad[2][e]),
+                             silu_ref(z[e], tabs.exp2));
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {  // rows past n lie past the buffer's end: not stored
+        const int t = o * kFt + tw + e;
+        const unsigned at = o < 0 ? 0xfffffff0u : ((unsigned)t * (unsigned)di + (unsigned)idx) * 4u;
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(out[e]), rsrc, (int)at, 0, 0);
+      }
+      __syncthreads();
+    }
+  }
+}
+
+// the fused kernel's shapes: whole 16-channel groups per head, and y and proj
+// (the wider) within the bounds-checked buffers' 32-bit offsets, tiles past
+// the end included
+inline bool ssm_fused_fits(int n, int pd, int hd) {
+  return hd % kFc == 0 && ((size_t)n + 4 * kFt) * pd * 4 < 0xf0000000u;
 }
 
 __global__ void k_advance_pos(int* ctl, int n) {
@@ -634,8 +830,9 @@ int ensure_prefill(bm_hip_model* m, int n) {
   MCHECK(hipMalloc(&m->pact, (size_t)n * bm::act_row_bytes((int)K)));
   MCHECK(hipMalloc(&m->pxq, (size_t)n * K));
   MCHECK(hipMalloc(&m->ptok, (size_t)n * 4));
-  MCHECK(hipMalloc(&m->ppre,
-                   bm::pre_layout(n < bm::kSsmChunk ? n : bm::kSsmChunk, m->di, m->nh).total * 4));
+  if (!bm::ssm_fused_fits(n, m->pd, m->hd))
+    MCHECK(hipMalloc(&m->ppre,
+                     bm::pre_layout(n < bm::kSsmChunk ? n : bm::kSsmChunk, m->di, m->nh).total * 4));
   m->pcap = n;  // only once every buffer exists
   return 0;
 }
@@ -912,14 +1109,21 @@ extern "C" int bm_hip_model_prefill(bm_hip_model_t* m, const int32_t* tokens, in
   MCHECK(hipGetLastError());
   for (int l = 0; l < m->nl; ++l) {
     const Layer& Ly = m->L[l];
-    // block_step_batch (src/block.c:378-447): batched in_proj, the SSM in
-    // three phases per chunk of tokens (k_ssm_prep, k_ssm_scan, k_ssm_out),
-    // batched out_proj, then x += out (src/model.c:1139-1142)
+    // block_step_batch (src/block.c:378-447): batched in_proj, the SSM in one
+    // kernel (k_ssm_fused) or, for head dims it does not take, in three phases
+    // per chunk of tokens (k_ssm_prep, k_ssm_scan, k_ssm_out), batched
+    // out_proj, then x += out (src/model.c:1139-1142)
     if (bitlinear(m, m->px, n, dm, Ly.in_norm, Ly.in_proj, m->pd, Ly.in_scale, m->pproj,
                   bm::MODE_STORE, m->pact, m->pscale, m->pxq, s))
       return -1;
     float* cs = m->conv_state + (size_t)l * 3 * di;
-    for (int t0 = 0; t0 < n; t0 += bm::kSsmChunk) {
+    if (bm::ssm_fused_fits(n, m->pd, m->hd)) {
+      hipLaunchKernelGGL(bm::k_ssm_fused, dim3(di / bm::kFc), dim3(64 * (bm::kFtasks + 2)), 0, s,
+                         m->pproj, m->pd, n, di, m->hd, Ly.dt_bias, Ly.A, Ly.conv_wt, Ly.conv_b,
+                         cs, m->ssm_state + (size_t)l * di, Ly.D, m->ctl, m->py);
+      MCHECK(hipGetLastError());
+    }
+    for (int t0 = bm::ssm_fused_fits(n, m->pd, m->hd) ? n : 0; t0 < n; t0 += bm::kSsmChunk) {
       const int nt = n - t0 < bm::kSsmChunk ? n - t0 : bm::kSsmChunk;
       const bm::PreLayout PL = bm::pre_layout(nt, di, m->nh);
       hipLaunchKernelGGL(bm::k_ssm_prep, dim3((di + 255) / 256, PL.nqr), dim3(256), 0, s,
