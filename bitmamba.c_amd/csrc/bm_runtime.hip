@@ -43,6 +43,42 @@ extern "C" const char* bm_hip_last_error(void) { return g_err; }
 constexpr size_t kScratchBytes = (size_t)8 << 20;
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
+namespace bm {
+
+// up to three runs of bytes at the same offsets of a device buffer and of
+// mapped host memory, in slices of `slice` bytes, a block each
+struct HostSlices {
+  size_t off[3], bytes[3], slice;
+  int first[3];  // the run's first block
+};
+
+__global__ __launch_bounds__(256) void k_to_host(HostSlices h, const uint8_t* __restrict__ src,
+                                                 uint8_t* __restrict__ dst,
+                                                 unsigned* __restrict__ flags, unsigned seq) {
+  const int b = blockIdx.x;
+  const int i = b >= h.first[2] ? 2 : (b >= h.first[1] ? 1 : 0);
+  const size_t at = (size_t)(b - h.first[i]) * h.slice;
+  const size_t n = min(h.slice, h.bytes[i] - at), base = h.off[i] + at;
+  const uint8_t* __restrict__ p = src + base;
+  uint8_t* __restrict__ q = dst + base;
+  if (((uintptr_t)p | (uintptr_t)q) % 16 == 0) {
+    const size_t n16 = n / 16;
+#pragma unroll 4
+    for (size_t k = threadIdx.x; k < n16; k += 256) ((uint4*)q)[k] = ((const uint4*)p)[k];
+    for (size_t k = 16 * n16 + threadIdx.x; k < n; k += 256) q[k] = p[k];
+  } else {
+    for (size_t k = threadIdx.x; k < n; k += 256) q[k] = p[k];
+  }
+  // each wave waits for its own stores (the barrier does not), then the
+  // release writes back what L2 holds of them before the word
+  __asm__ __volatile__("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(flags + b, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+}  // namespace bm
+
 namespace {
 
 constexpr int kMaxDevices = 16;
@@ -117,10 +153,18 @@ bool ensure_dev(DevBuf& b, size_t bytes) {
 bool ensure_pinned(DevBuf& b, size_t bytes) {
   if (b.bytes >= bytes && b.ptr) return true;
   if (b.ptr) (void)hipHostFree(b.ptr);
-  b.ptr = nullptr;
-  b.bytes = 0;
+  b = DevBuf{};
   size_t want = bytes < 65536 ? 65536 : bytes + bytes / 4;
-  BM_HIP_CHECK_RET(hipHostMalloc(&b.ptr, want, hipHostMallocDefault), false);
+  void* p = nullptr;
+  BM_HIP_CHECK_RET(hipHostMalloc(&p, want, hipHostMallocMapped | hipHostMallocCoherent), false);
+  void* d = nullptr;
+  if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) {
+    (void)hipHostFree(p);
+    bm_set_error("hipHostGetDevicePointer failed");
+    return false;
+  }
+  b.ptr = p;
+  b.dev = d;
   b.bytes = want;
   return true;
 }
@@ -371,6 +415,47 @@ void bitlinear_check(int n, const struct tensor* w) {
   }
 }
 
+struct OutPart {
+  size_t off, bytes;  // the same offset in the device buffer and the stage
+};
+
+// The results of a host-pointer call: a kernel copies them to the stage (the
+// caller's `out` first, part 0) in slices, a block each, and publishes every
+// slice, so that the CPU copies one to `out` while the next ones travel; no
+// copy commands, events or stream wait.  Bound by the bus and the CPU's one
+// copying thread: 256 tokens, K = 1024 -> 4192 (4.3 MB of results) 330 -> 258
+// us per call against one copy command, a wait and one copy by the CPU; copy
+// commands in 512 KiB pieces with an event each were no faster than that.
+hipError_t results_to_host(Backend& b, const OutPart (&part)[3], uint8_t* out, uint8_t* hs,
+                           const uint8_t* dev, hipStream_t s) {
+  // 64 KiB slices, more where that would take more blocks than words
+  size_t slice = 64 * 1024, total = 0;
+  for (const OutPart& p : part) total += p.bytes;
+  while ((total + slice - 1) / slice + 3 > (size_t)kDropInMaxBlocks) slice *= 2;
+  bm::HostSlices hsl{};
+  int blocks = 0;
+  for (int i = 0; i < 3; ++i) {
+    hsl.off[i] = part[i].off;
+    hsl.bytes[i] = part[i].bytes;
+    hsl.first[i] = blocks;
+    blocks += (int)((part[i].bytes + slice - 1) / slice);
+  }
+  hsl.slice = slice;
+  const unsigned seq = next_seq(b);
+  hipLaunchKernelGGL(bm::k_to_host, dim3(blocks), dim3(256), 0, s, hsl, dev,
+                     (uint8_t*)b.h_stage.dev, (unsigned*)b.h_flag.dev, seq);
+  hipError_t e = hipGetLastError();
+  const unsigned* flags = (const unsigned*)b.h_flag.ptr;
+  for (int k = 0; k < blocks && e == hipSuccess; ++k) {
+    e = wait_flags(flags + k, 1, seq, s);
+    const size_t off = (size_t)k * slice;
+    if (e == hipSuccess && off < part[0].bytes)
+      memcpy(out + off, hs + part[0].off + off,
+             part[0].bytes - off < slice ? part[0].bytes - off : slice);
+  }
+  return e;
+}
+
 // Host-pointer batch BitLinear: quantize + product on the device, results
 // copied back.  Any HIP failure is fatal (never zero outputs silently).
 void host_bitlinear(const float* x, int M, int n, const uint8_t* packed, int rows, int cols,
@@ -397,6 +482,7 @@ void host_bitlinear(const float* x, int M, int n, const uint8_t* packed, int row
       !ensure_dev(b.d_act, abytes) || !ensure_dev(b.d_scale, (size_t)M * 4))
     die("scratch allocation");
   if (!ensure_pinned(b.h_stage, xbytes > iobytes ? xbytes : iobytes)) die("pinned staging");
+  if (!ensure_dropin(b)) die("completion words");
 
   // small calls: [x | out | x_norm | int8] in mapped host memory, no copies
   const size_t o_x = bm::align_up(iobytes, 256);
@@ -406,11 +492,18 @@ void host_bitlinear(const float* x, int M, int n, const uint8_t* packed, int row
   const float* dx = zc ? (const float*)(dio + o_x) : (const float*)b.d_x.ptr;
   hipStream_t s = b.stream;
   hipError_t e = hipSuccess;
+  bool out_done = false;
   if (zc) {
     memcpy(hs + o_x, x, xbytes);
   } else {
     memcpy(hs, x, xbytes);
-    e = hipMemcpyAsync(b.d_x.ptr, hs, xbytes, hipMemcpyHostToDevice, s);
+    // the quantizers read x once: straight from the stage (258 against 284 us
+    // per call of 256 tokens with a copy command; n > 8192 takes a quantizer
+    // that reads it three times)
+    if (n <= 8192)
+      dx = (const float*)b.h_stage.dev;
+    else
+      e = hipMemcpyAsync(b.d_x.ptr, hs, xbytes, hipMemcpyHostToDevice, s);
   }
   const bool generic = bm::product_needs_generic(M, cols);
   const int nblk = M == 1 && bm::rows_fit(n) ? bm::dropin_blocks(rows, n) : 0;
@@ -435,14 +528,21 @@ void host_bitlinear(const float* x, int M, int n, const uint8_t* packed, int row
         e = bm::launch_product((const uint8_t*)b.d_act.ptr, (const float*)b.d_scale.ptr, M, dW,
                                rows, cols, w_scale, true, dio, bm::MODE_STORE, s);
     }
-    if (e == hipSuccess && !zc) e = hipMemcpyAsync(hs, dio, iobytes, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e == hipSuccess && !zc) {
+      // x_norm leaves for the last token only
+      const size_t last = o_norm + (size_t)(M - 1) * n * sizeof(float);
+      const OutPart part[3] = {{0, obytes}, {last, x_norm_buf ? (size_t)n * 4 : 0},
+                               {o_q, x_quant ? qbytes : 0}};
+      e = results_to_host(b, part, (uint8_t*)out, hs, dio, s);
+      out_done = e == hipSuccess;
+    }
+    if (e == hipSuccess && !out_done) e = hipStreamSynchronize(s);
   }
   if (e != hipSuccess) {
     bm_set_error("%s", hipGetErrorString(e));
     die("bitlinear");
   }
-  memcpy(out, hs, obytes);
+  if (!out_done) memcpy(out, hs, obytes);
   // x_norm_buf is a single n-vector reused per token: the last token stays
   if (x_norm_buf)
     memcpy(x_norm_buf, hs + o_norm + (size_t)(M - 1) * n * sizeof(float), (size_t)n * 4);
