@@ -50,17 +50,20 @@ inline constexpr uint64_t kExp2Tab[32] = {
 
 // tab: kExp2Tab or a copy of it
 BM_HD float expf_tab(float x, const uint64_t* tab) {
-  // special cases (selected at the end, no branches): overflow above
-  // ~88.72, underflow to 0 below ~-103.97, NaN passes through
-  const bool nan = x != x;
-  const bool ovf = x > 0x1.62e42ep6f;
-  const bool unf = x < -0x1.9fe368p6f;
+  // overflow (above ~88.72) and underflow to 0 (below ~-103.97) come out of
+  // the final rounding to float once x is clamped a little beyond them; NaN
+  // passes through
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float xc = __builtin_amdgcn_fmed3f(x, -150.0f, 90.0f);
+#else
+  const float xc = x < -150.0f ? -150.0f : (x > 90.0f ? 90.0f : x);
+#endif
   const double InvLn2N = 0x1.71547652b82fep+0 * 32;
   const double Shift = 0x1.8p+52;
   const double C0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32;
   const double C1 = 0x1.ebfce50fac4f3p-3 / 32 / 32;
   const double C2 = 0x1.62e42ff0c52d6p-1 / 32;
-  const double xd = (double)((nan || ovf || unf) ? 0.0f : x);
+  const double xd = (double)xc;
   // x*32/ln2 = k + r, |r| <= 1/2
   double kd = __builtin_fma(InvLn2N, xd, Shift);
   const uint64_t ki = u64_of(kd);
@@ -74,10 +77,7 @@ BM_HD float expf_tab(float x, const uint64_t* tab) {
   double y = __builtin_fma(C2, r, 1.0);
   y = __builtin_fma(z, r2, y);
   y = y * s;
-  float res = (float)y;
-  res = unf ? 0.0f : res;
-  res = ovf ? __builtin_inff() : res;
-  return nan ? x : res;
+  return x != x ? x : (float)y;
 }
 BM_HD float expf_glibc(float x) { return expf_tab(x, kExp2Tab); }
 

@@ -275,16 +275,19 @@ __global__ __launch_bounds__(256) void k_ssm_out(const float* __restrict__ pre,
 // three-phase version's planes nothing goes through memory.  A tile's inputs
 // are loaded one iteration ahead; loads and stores are unconditional (through
 // bounds-checked buffers) so that a wait covers only what it needs.  Tokens past n carry decay 1 and xa * B * dt = -0.
-// Bound by instruction issue: the SIMDs that hold wave 0 and wave 1 beside two
-// task waves issue ~650 vector instructions per tile (silu ~55 each).  1B
-// shape, 1024 tokens, per layer: 23.7 us against 17.6 + 13.9 + 13.9 us for
-// the three kernels (the planes were ~130 MB of traffic); the prefill of 1024
-// tokens 2.515 -> 1.854 ms, of 8 tokens 0.917 -> 0.663 ms, with the
-// quantizers' change in both.  With plain loads whose row or ring address is
-// chosen per lane (a branch around each) 27.3 us.
-constexpr int kFc = 16, kFt = 64, kFtasks = 8;  // channels, tile, task waves
+// What bounds it: ~1.1 us per tile, the task waves' dependent fp64 chains (two
+// silu deep, ~220 instructions per wave and tile, two task waves per SIMD).
+// Tried without gain: task waves moved off the SIMDs of waves 0 and 1 (12
+// waves, two idle), inputs loaded two iterations ahead (23.1 us), the decay
+// of a tile one iteration after its dt.  1B shape, 1024 tokens, per layer:
+// 22 us (27.3 with plain loads whose row or ring address is chosen per lane,
+// a branch around each; 23.9 with the recurrence reading each quad as it
+// comes) against 17.6 + 13.9 + 13.9 us for the three kernels, whose planes
+// were ~130 MB of traffic.  The prefill of 1024 tokens 2.46 -> 1.77 ms, of 8
+// tokens 0.92 -> 0.65 ms, with the quantizers' change in both.
+constexpr int kFc = 16, kFt = 64, kFwaves = 10;  // channels, tokens per tile, waves
 
-__global__ __launch_bounds__(64 * (kFtasks + 2)) void k_ssm_fused(
+__global__ __launch_bounds__(64 * kFwaves) void k_ssm_fused(
     const float* __restrict__ proj, int pd, int n, int di, int hd,
     const float* __restrict__ dt_bias, const float* __restrict__ A, const float* __restrict__ cw,
     const float* __restrict__ cb, float* __restrict__ cs, float* __restrict__ ssm,
@@ -313,19 +316,27 @@ __global__ __launch_bounds__(64 * (kFtasks + 2)) void k_ssm_fused(
     __syncthreads();
     for (int it = 0; it < nt + 3; ++it) {
       const int k = it - 2;
-      if (k >= 0 && k < nt) {
+      if (k >= 0 && k < nt && lane < kFc) {
         const float* __restrict__ xb = s_xb[k & 1] + c * ROW;
         const float* __restrict__ dec = s_dec[k & 3];
         float* __restrict__ o = s_st[k & 1] + c * ROW;
+        // all of the tile's operands first: a quad's dependent adds take
+        // ~40 cycles, less than an LDS round trip
+        float4 x[kFt / 4], d[kFt / 4];
 #pragma unroll
-        for (int q = 0; q < kFt; q += 4) {
-          const float4 x = *(const float4*)(xb + q), d = *(const float4*)(dec + q);
+        for (int q = 0; q < kFt / 4; ++q) {
+          d[q] = *(const float4*)(dec + 4 * q);
+          x[q] = *(const float4*)(xb + 4 * q);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < kFt / 4; ++q) {
           float4 r;
-          r.x = __fadd_rn(__fmul_rn(st, d.x), x.x);
-          r.y = __fadd_rn(__fmul_rn(r.x, d.y), x.y);
-          r.z = __fadd_rn(__fmul_rn(r.y, d.z), x.z);
-          st = r.w = __fadd_rn(__fmul_rn(r.z, d.w), x.w);
-          if (lane < kFc) *(float4*)(o + q) = r;
+          r.x = __fadd_rn(__fmul_rn(st, d[q].x), x[q].x);
+          r.y = __fadd_rn(__fmul_rn(r.x, d[q].y), x[q].y);
+          r.z = __fadd_rn(__fmul_rn(r.y, d[q].z), x[q].z);
+          st = r.w = __fadd_rn(__fmul_rn(r.z, d[q].w), x[q].w);
+          *(float4*)(o + 4 * q) = r;
         }
       }
       __syncthreads();
@@ -1166,7 +1177,7 @@ static int enqueue_prefill(bm_hip_model* m, const int32_t* tokens, int n) {
       return -1;
     float* cs = m->conv_state + (size_t)l * 3 * di;
     if (bm::ssm_fused_fits(n, m->pd, m->hd)) {
-      hipLaunchKernelGGL(bm::k_ssm_fused, dim3(di / bm::kFc), dim3(64 * (bm::kFtasks + 2)), 0, s,
+      hipLaunchKernelGGL(bm::k_ssm_fused, dim3(di / bm::kFc), dim3(64 * bm::kFwaves), 0, s,
                          m->pproj, m->pd, n, di, m->hd, Ly.dt_bias, Ly.A, Ly.conv_wt, Ly.conv_b,
                          cs, m->ssm_state + (size_t)l * di, Ly.D, m->ctl, m->py);
       MCHECK(hipGetLastError());
