@@ -125,6 +125,7 @@ constexpr int kCandLds = 512;      // candidates kept in LDS when they fit
 constexpr int kListsPerWave = kFront / (kThreads / 64);
 
 constexpr int kSortMax = 4096;  // entries sorted in LDS by the draw without top-k
+constexpr int kRankMax = 256;   // of them, by rank instead of a bitonic network
 
 struct Smem {
   union {
@@ -643,7 +644,8 @@ __device__ void embed_next(int token, const StepIO& io) {
 // sequential code below runs.  So does it where more than kSortMax entries
 // share the bucket that decides, and for a top_k that cuts (above 256).
 // V = 50257, logits of spread 4 at temp = 0.8, top_p = 0.9: 2759 us per call
-// in turn on one thread (the sum, then the heap), 53.6 us this way.
+// in turn on one thread (the sum, then the heap), 52 us this way (55.9 with a
+// bitonic network for any count).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double wave_sum_f64(double v) {  // the same bits in every lane
 #pragma unroll
@@ -730,6 +732,19 @@ __device__ int sort_buckets(const Scratch& sc, const int (&pc)[kListsPerWave], i
   }
   __syncthreads();
   const int n = min(uni(sm.iwork[6]), kSortMax);
+  if (n <= kRankMax) {  // few: each key's rank by comparing it with all
+    uint64_t own = 0;
+    int r = 0;
+    if ((int)threadIdx.x < n) {
+      own = sm.keys[threadIdx.x];
+#pragma unroll 4
+      for (int i = 0; i < n; ++i) r += sm.keys[i] < own;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < n) sm.keys[r] = own;
+    __syncthreads();
+    return n;
+  }
   int size = 64;
   while (size < n) size *= 2;
   for (int i = n + threadIdx.x; i < size; i += kThreads) sm.keys[i] = ~0ull;
@@ -802,10 +817,11 @@ __device__ int find_key(int n, double base, double x, double slack, bool first, 
 template <bool INCL>
 __device__ int find_bucket(const double (&s)[2], const int (&c)[2], double x, double* sum, int* cnt,
                            Smem& sm) {
-  double sb;
+  // counts below 2^53 add exactly as doubles
+  double sb, cb_d;
   block_scan_f64(s[0] + s[1], &sb, sm);
-  unsigned total;
-  const int cb = (int)block_scan((unsigned)(c[0] + c[1]), sm, &total);
+  block_scan_f64((double)(c[0] + c[1]), &cb_d, sm);
+  const int cb = (int)cb_d;
   if (threadIdx.x == 0) sm.iwork[7] = kPBuckets;
   __syncthreads();
   const double r0 = sb + s[0], r1 = r0 + s[1];
