@@ -644,14 +644,33 @@ __device__ void embed_next(int token, const StepIO& io) {
 // sequential code below runs.  So does it where more than kSortMax entries
 // share the bucket that decides, and for a top_k that cuts (above 256).
 // V = 50257, logits of spread 4 at temp = 0.8, top_p = 0.9: 2759 us per call
-// in turn on one thread (the sum, then the heap), 52 us this way (55.9 with a
-// bitonic network for any count).
+// in turn on one thread (the sum, then the heap), 48 us this way (52 with LDS
+// shuffles in the scans, 55.9 with a bitonic network for any count too).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double wave_sum_f64(double v) {  // the same bits in every lane
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+// prefix sums over the wave on DPP (a shuffle through LDS per step costs
+// several times as much)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f64(double v) {  // lanes without a source get 0
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)dpp_or0<CTRL, ROWS>((int)(uint32_t)u);
+  const uint32_t hi = (uint32_t)dpp_or0<CTRL, ROWS>((int)(uint32_t)(u >> 32));
+  return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
 }
+__device__ __forceinline__ double wave_scan_f64(double v) {
+  v += dpp_f64<0x111, 0xf>(v);
+  v += dpp_f64<0x112, 0xf>(v);
+  v += dpp_f64<0x114, 0xf>(v);
+  v += dpp_f64<0x118, 0xf>(v);
+  v += dpp_f64<0x142, 0xa>(v);
+  return v + dpp_f64<0x143, 0xc>(v);
+}
+__device__ __forceinline__ double lane_f64(double v, int lane) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+  return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+__device__ __forceinline__ double wave_sum_f64(double v) { return lane_f64(wave_scan_f64(v), 63); }
 
 // every thread has the same v: make the branches on it uniform (barriers
 // follow on both sides of them)
@@ -677,19 +696,17 @@ __device__ __forceinline__ bool softmax_scale(double sum, int n, float* inv) {
 // block-wide inclusive prefix sum; *before = the sum in front of the thread
 __device__ double block_scan_f64(double v, double* before, Smem& sm) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  double incl = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const double u = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += u;
-  }
+  const double incl = wave_scan_f64(v);
   __syncthreads();
   if (lane == 63) sm.dscan[wave] = incl;
   __syncthreads();
   double off = 0.0;
-  for (int w = 0; w < wave; ++w) off += sm.dscan[w];
-  const double up = __shfl_up(incl, 1, 64);
-  *before = lane ? off + up : off;
+#pragma unroll
+  for (int w = 0; w < kThreads / 64; ++w) {  // all loads at once
+    const double t = sm.dscan[w];
+    off += w < wave ? t : 0.0;
+  }
+  *before = off + dpp_f64<0x138, 0xf>(incl);
   return off + incl;
 }
 
@@ -858,17 +875,12 @@ __device__ bool draw_parallel(const Scratch& sc, const int (&pc)[kListsPerWave],
     // in index order: the list, then the entry the walk ends at
     if (!sure_float(total, n, &f)) return false;
     const double r = (double)__fmul_rn(rng_float(g), f);
-    double incl = ps;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const double u = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += u;
-    }
+    const double incl = wave_scan_f64(ps);
     const uint64_t hit = __ballot(mine > 0 && incl > r);
     if (!hit) return false;
     const int l = __ffsll((unsigned long long)hit) - 1;
-    const double base = l ? __shfl(incl, l - 1, 64) : 0.0;
-    const int cnt = __shfl(mine, l, 64);
+    const double base = l ? lane_f64(incl, l - 1) : 0.0;
+    const int cnt = __builtin_amdgcn_readlane(mine, l);
     const size_t at = (size_t)l * seg;
     static_assert(kMaxVocab / kFront + 4 <= 4 * kThreads, "a list fits one pass");
     double v[4], own = 0.0, before;
@@ -1014,6 +1026,7 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_scale(float* __restrict_
 // histogram over logits >= the min_p threshold (src/model.c:180-194) and
 // writes its pre-candidates: (i, logits[i]) with logits[i] >= the lowest
 // extraction threshold, in index order, to pre[block * seg ..].
+template <bool TOPK>
 __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __restrict__ logits,
                                                              int V, SampleParams p,
                                                              void* scratch,
@@ -1030,8 +1043,7 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __rest
   const float4 q = load4(logits, i0 + 4 * (int)threadIdx.x, i1);  // before the max: independent
   const float max_logit = front_max(pmax, npart);
   const float min_p_thresh = min_p_threshold(max_logit, p.min_p);
-  const int eff_k = effective_k(p.top_k);
-  const bool use_hist = eff_k > 0;
+  constexpr bool use_hist = TOPK;
   const float bucket_scale = bucket_scale_of();
   const float pre_thresh =
       use_hist ? extract_threshold(max_logit, min_p_thresh, kBuckets - 1) : min_p_thresh;
@@ -1164,6 +1176,9 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_probs(int V, void* scrat
 // lists in order, selection, softmax, sorting and the draw; then the step
 // bookkeeping and the next token's embedding (StepIO).  Leaves the
 // histogram cleared for the next call.
+// TOPK: an effective top-k; separate kernels, since the two ways share little
+// and the larger one's registers cost the other 2.4 of 20.6 us per call.
+template <bool TOPK>
 __global__ __launch_bounds__(1024) void k_sample(const float* __restrict__ logits, int V,
                                                  SampleParams p, uint64_t* __restrict__ rng_state,
                                                  void* scratch, const float* __restrict__ pmax,
@@ -1185,11 +1200,10 @@ __global__ __launch_bounds__(1024) void k_sample(const float* __restrict__ logit
   uint64_t rng = *rng_state;
   const float max_logit = front_max(pmax, npart);
   const float min_p_thresh = min_p_threshold(max_logit, p.min_p);
-  const int eff_k = effective_k(p.top_k);
   int token = 0;
   Cand* probs = sc.probs;
-  Cand* probs2 = sc.pre;  // free once the candidates are gathered
-  if (eff_k > 0) {
+  if constexpr (TOPK) {
+    const int eff_k = effective_k(p.top_k);
     // the cutoff bucket (src/model.c:196-213): first bucket whose running
     // count reaches k; lane l of wave 0 holds buckets 2l, 2l+1
     if (threadIdx.x < 64) {
@@ -1251,6 +1265,7 @@ __global__ __launch_bounds__(1024) void k_sample(const float* __restrict__ logit
     }
   } else if (!draw_parallel(sc, pc, seg, p, rng, &token, sm)) {
     // no top-k: every candidate over the min_p threshold (src/model.c:278-300)
+    Cand* probs2 = sc.pre;  // free once the candidates are gathered
     int n = gather(sc, pc, seg, min_p_thresh, sc.probs, &probs, sm);
     if (n == 0) {
       token = argmax_scan(logits, V, logits[0], sm);
@@ -1361,13 +1376,19 @@ hipError_t launch_sample(float* logits, int V, float temp, float min_p, float to
     pmax = scratch_of(scratch, V).pmax;
     npart = kFront;
   }
-  hipLaunchKernelGGL(k_samp_hist, dim3(kFront), dim3(kFrontThreads), 0, s, logits, V, p, scratch,
-                     pmax, npart, gated ? (const int*)ctl : nullptr);
-  if (effective_k(top_k) == 0)
-    hipLaunchKernelGGL(k_samp_probs, dim3(kFront), dim3(kFrontThreads), 0, s, V, scratch,
-                       gated ? (const int*)ctl : nullptr);
-  hipLaunchKernelGGL(k_sample, dim3(1), dim3(kThreads), 0, s, logits, V, p, rng_state, scratch,
-                     pmax, npart, io);
+  const int* gate = gated ? (const int*)ctl : nullptr;
+  const dim3 front(kFront), ft(kFrontThreads), one(1), all(kThreads);
+  if (effective_k(top_k) > 0) {
+    hipLaunchKernelGGL(k_samp_hist<true>, front, ft, 0, s, logits, V, p, scratch, pmax, npart, gate);
+    hipLaunchKernelGGL(k_sample<true>, one, all, 0, s, logits, V, p, rng_state, scratch, pmax, npart,
+                       io);
+  } else {
+    hipLaunchKernelGGL(k_samp_hist<false>, front, ft, 0, s, logits, V, p, scratch, pmax, npart,
+                       gate);
+    hipLaunchKernelGGL(k_samp_probs, front, ft, 0, s, V, scratch, gate);
+    hipLaunchKernelGGL(k_sample<false>, one, all, 0, s, logits, V, p, rng_state, scratch, pmax,
+                       npart, io);
+  }
   return hipGetLastError();
 }
 
