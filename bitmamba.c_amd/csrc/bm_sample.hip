@@ -12,7 +12,7 @@
 //                 lowest threshold the extraction can use (the histogram's
 //                 last bucket, or the min_p threshold), a superset of the
 //                 candidates.
-//   k_samp_probs  (no top-k) the probabilities, and per value bucket their
+//   k_samp_probs  (no top-k, see tries_parallel) the probabilities, and per value bucket their
 //                 count and sum.
 // k_sample then runs the rest on one 1024-thread block: the cutoff bucket,
 // the candidates filtered from the pre-candidate lists in order, selection,
@@ -197,6 +197,13 @@ __device__ __forceinline__ float min_p_threshold(float max_logit, float min_p) {
 
 __host__ __device__ __forceinline__ int effective_k(int top_k) {
   return (top_k > 0 && top_k <= 256) ? top_k : 0;  // src/model.c:168-170
+}
+
+// Without top-k: whether draw_parallel is tried.  Not where min_p alone cuts
+// (top_p >= 1): it leaves few candidates, which one thread walks in 16 us per
+// call, 19 with the probabilities' launch and the buckets.
+__host__ __device__ __forceinline__ bool tries_parallel(const SampleParams& p) {
+  return p.top_p < 1.0f || !(p.min_p > 0.0f);
 }
 
 __device__ __forceinline__ float bucket_scale_of() {
@@ -1044,6 +1051,7 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __rest
   const float max_logit = front_max(pmax, npart);
   const float min_p_thresh = min_p_threshold(max_logit, p.min_p);
   constexpr bool use_hist = TOPK;
+  const bool exps = !TOPK && tries_parallel(p);
   const float bucket_scale = bucket_scale_of();
   const float pre_thresh =
       use_hist ? extract_threshold(max_logit, min_p_thresh, kBuckets - 1) : min_p_thresh;
@@ -1051,7 +1059,7 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __rest
   __shared__ double wsum[NW];
   // k_samp_probs adds to the buckets after this kernel
   constexpr int kClear = kPBuckets / kFront;
-  if (!use_hist && threadIdx.x < kClear) {
+  if (exps && threadIdx.x < kClear) {
     sc.bsum[blockIdx.x * kClear + threadIdx.x] = 0.0;
     sc.bcnt[blockIdx.x * kClear + threadIdx.x] = 0;
   }
@@ -1106,7 +1114,7 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __rest
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       if (h[e]) {
-        if (!use_hist) {  // the softmax numerator (src/model.c:292-297)
+        if (exps) {  // the softmax numerator (src/model.c:292-297)
           const float ex = libm::expf_glibc(__fsub_rn(v[e], max_logit));
           pv[pos] = ex;
           esum += (double)ex;
@@ -1115,7 +1123,7 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __rest
       }
     off += row;
   }
-  if (!use_hist) {
+  if (exps) {
     esum = wave_sum_f64(esum);
     if (lane == 0) wsum[wave] = esum;
     __syncthreads();
@@ -1263,7 +1271,7 @@ __global__ __launch_bounds__(1024) void k_sample(const float* __restrict__ logit
       }
       token = filter_and_sample(src, n, p.top_p, 0, rng, sm);
     }
-  } else if (!draw_parallel(sc, pc, seg, p, rng, &token, sm)) {
+  } else if (!tries_parallel(p) || !draw_parallel(sc, pc, seg, p, rng, &token, sm)) {
     // no top-k: every candidate over the min_p threshold (src/model.c:278-300)
     Cand* probs2 = sc.pre;  // free once the candidates are gathered
     int n = gather(sc, pc, seg, min_p_thresh, sc.probs, &probs, sm);
@@ -1385,7 +1393,8 @@ hipError_t launch_sample(float* logits, int V, float temp, float min_p, float to
   } else {
     hipLaunchKernelGGL(k_samp_hist<false>, front, ft, 0, s, logits, V, p, scratch, pmax, npart,
                        gate);
-    hipLaunchKernelGGL(k_samp_probs, front, ft, 0, s, V, scratch, gate);
+    if (tries_parallel(p))
+      hipLaunchKernelGGL(k_samp_probs, front, ft, 0, s, V, scratch, gate);
     hipLaunchKernelGGL(k_sample<false>, one, all, 0, s, logits, V, p, rng_state, scratch, pmax,
                        npart, io);
   }
