@@ -1033,7 +1033,7 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_scale(float* __restrict_
 // histogram over logits >= the min_p threshold (src/model.c:180-194) and
 // writes its pre-candidates: (i, logits[i]) with logits[i] >= the lowest
 // extraction threshold, in index order, to pre[block * seg ..].
-template <bool TOPK>
+template <bool TOPK, bool PAR>
 __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __restrict__ logits,
                                                              int V, SampleParams p,
                                                              void* scratch,
@@ -1051,7 +1051,7 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __rest
   const float max_logit = front_max(pmax, npart);
   const float min_p_thresh = min_p_threshold(max_logit, p.min_p);
   constexpr bool use_hist = TOPK;
-  const bool exps = !TOPK && tries_parallel(p);
+  constexpr bool exps = !TOPK && PAR;  // tries_parallel
   const float bucket_scale = bucket_scale_of();
   const float pre_thresh =
       use_hist ? extract_threshold(max_logit, min_p_thresh, kBuckets - 1) : min_p_thresh;
@@ -1184,9 +1184,10 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_probs(int V, void* scrat
 // lists in order, selection, softmax, sorting and the draw; then the step
 // bookkeeping and the next token's embedding (StepIO).  Leaves the
 // histogram cleared for the next call.
-// TOPK: an effective top-k; separate kernels, since the two ways share little
-// and the larger one's registers cost the other 2.4 of 20.6 us per call.
-template <bool TOPK>
+// TOPK: an effective top-k; PAR: without one, tries_parallel.  Separate
+// kernels, since the ways share little and the largest one's registers cost
+// the others ~2 of 16 to 20 us per call.
+template <bool TOPK, bool PAR>
 __global__ __launch_bounds__(1024) void k_sample(const float* __restrict__ logits, int V,
                                                  SampleParams p, uint64_t* __restrict__ rng_state,
                                                  void* scratch, const float* __restrict__ pmax,
@@ -1271,7 +1272,10 @@ __global__ __launch_bounds__(1024) void k_sample(const float* __restrict__ logit
       }
       token = filter_and_sample(src, n, p.top_p, 0, rng, sm);
     }
-  } else if (!tries_parallel(p) || !draw_parallel(sc, pc, seg, p, rng, &token, sm)) {
+  } else {
+    bool drawn = false;
+    if constexpr (PAR) drawn = draw_parallel(sc, pc, seg, p, rng, &token, sm);
+    if (!drawn) {
     // no top-k: every candidate over the min_p threshold (src/model.c:278-300)
     Cand* probs2 = sc.pre;  // free once the candidates are gathered
     int n = gather(sc, pc, seg, min_p_thresh, sc.probs, &probs, sm);
@@ -1322,6 +1326,7 @@ __global__ __launch_bounds__(1024) void k_sample(const float* __restrict__ logit
         sort_large(probs, probs2, n, sm);
         token = filter_and_sample(probs, n, p.top_p, p.top_k, rng, sm);
       }
+    }
     }
   }
 
@@ -1387,16 +1392,21 @@ hipError_t launch_sample(float* logits, int V, float temp, float min_p, float to
   const int* gate = gated ? (const int*)ctl : nullptr;
   const dim3 front(kFront), ft(kFrontThreads), one(1), all(kThreads);
   if (effective_k(top_k) > 0) {
-    hipLaunchKernelGGL(k_samp_hist<true>, front, ft, 0, s, logits, V, p, scratch, pmax, npart, gate);
-    hipLaunchKernelGGL(k_sample<true>, one, all, 0, s, logits, V, p, rng_state, scratch, pmax, npart,
-                       io);
+    hipLaunchKernelGGL((k_samp_hist<true, false>), front, ft, 0, s, logits, V, p, scratch, pmax,
+                       npart, gate);
+    hipLaunchKernelGGL((k_sample<true, false>), one, all, 0, s, logits, V, p, rng_state, scratch,
+                       pmax, npart, io);
+  } else if (tries_parallel(p)) {
+    hipLaunchKernelGGL((k_samp_hist<false, true>), front, ft, 0, s, logits, V, p, scratch, pmax,
+                       npart, gate);
+    hipLaunchKernelGGL(k_samp_probs, front, ft, 0, s, V, scratch, gate);
+    hipLaunchKernelGGL((k_sample<false, true>), one, all, 0, s, logits, V, p, rng_state, scratch,
+                       pmax, npart, io);
   } else {
-    hipLaunchKernelGGL(k_samp_hist<false>, front, ft, 0, s, logits, V, p, scratch, pmax, npart,
-                       gate);
-    if (tries_parallel(p))
-      hipLaunchKernelGGL(k_samp_probs, front, ft, 0, s, V, scratch, gate);
-    hipLaunchKernelGGL(k_sample<false>, one, all, 0, s, logits, V, p, rng_state, scratch, pmax,
-                       npart, io);
+    hipLaunchKernelGGL((k_samp_hist<false, false>), front, ft, 0, s, logits, V, p, scratch, pmax,
+                       npart, gate);
+    hipLaunchKernelGGL((k_sample<false, false>), one, all, 0, s, logits, V, p, rng_state, scratch,
+                       pmax, npart, io);
   }
   return hipGetLastError();
 }
