@@ -1068,6 +1068,10 @@ int load_into(bm_hip_model* m, const bm_bit2_view_t& v) {
 }
 
 int set_ctl(bm_hip_model* m, int token, const int* history, int history_len, int done = 0) {
+  if (history_len < 0) {  // would index the ring of tokens below its start
+    bm_set_error("negative history length %d", history_len);
+    return -1;
+  }
   // the history travels in the kernel's arguments: no copy, no wait
   bm::StartArgs a{};
   a.len = history_len < bm::kHistory ? history_len : bm::kHistory;

@@ -355,7 +355,8 @@ int bm_hip_model_reset(bm_hip_model_t *m);
 int bm_hip_model_prefill(bm_hip_model_t *m, const int32_t *tokens, int n);
 /* model_forward_step (src/model.c:1175-1314) with the sampler set by
  * bm_hip_model_set_sampler: returns the next token; history[history_len]
- * as the reference's caller keeps it (the last 256 tokens are used). */
+ * as the reference's caller keeps it (the last 256 tokens are used);
+ * -1 for a negative length. */
 int bm_hip_model_step(bm_hip_model_t *m,
                       int token,
                       const int *history,
