@@ -1160,6 +1160,17 @@ extern "C" int bm_hip_model_reset(bm_hip_model_t* m) {
   return 0;
 }
 
+// Nothing of a failed call runs on after it: the prompt is the caller's again,
+// and layer_state reads without waiting for the stream.  Relaxed: a caller
+// that is capturing another stream in this thread (which alone makes an
+// allocation or a wait here fail) would have this wait refused as well.
+static void wait_after_error(const bm_hip_model* m) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  (void)hipStreamSynchronize(m->stream);
+  if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+}
+
 // enqueues the prefill; `tokens` stays valid until the stream is waited for
 static int enqueue_prefill(bm_hip_model* m, const int32_t* tokens, int n) {
   if (n <= 0) return 0;
@@ -1213,7 +1224,10 @@ static int enqueue_prefill(bm_hip_model* m, const int32_t* tokens, int n) {
 }
 
 extern "C" int bm_hip_model_prefill(bm_hip_model_t* m, const int32_t* tokens, int n) {
-  if (enqueue_prefill(m, tokens, n)) return -1;
+  if (enqueue_prefill(m, tokens, n)) {
+    wait_after_error(m);
+    return -1;
+  }
   if (n > 0) MCHECK(hipStreamSynchronize(m->stream));
   return 0;
 }
@@ -1437,13 +1451,10 @@ extern "C" int bm_hip_model_set_layer_state(bm_hip_model_t* m, int layer, const 
   return 0;
 }
 
-extern "C" int bm_hip_model_generate(bm_hip_model_t* m, const int32_t* prompt, int n_prompt,
-                                     int n_steps, float penalty, int stop_on_eos,
-                                     int32_t* out_tokens, double* decode_ms) {
-  if (n_prompt <= 0 || n_steps < 0) {
-    bm_set_error("generate: empty prompt");
-    return -1;
-  }
+// generate after its argument check; on an error the stream may be busy
+static int generate_enqueued(bm_hip_model* m, const int32_t* prompt, int n_prompt, int n_steps,
+                             float penalty, int stop_on_eos, int32_t* out_tokens,
+                             double* decode_ms) {
   // src/main.c:451-500: prefill all but the last prompt token, history =
   // the prompt, then greedy steps from the last prompt token
   if (n_prompt > 1 && enqueue_prefill(m, prompt, n_prompt - 1)) return -1;
@@ -1466,6 +1477,19 @@ extern "C" int bm_hip_model_generate(bm_hip_model_t* m, const int32_t* prompt, i
         n = i + 1;
         break;
       }
+  return n;
+}
+
+extern "C" int bm_hip_model_generate(bm_hip_model_t* m, const int32_t* prompt, int n_prompt,
+                                     int n_steps, float penalty, int stop_on_eos,
+                                     int32_t* out_tokens, double* decode_ms) {
+  if (n_prompt <= 0 || n_steps < 0) {
+    bm_set_error("generate: empty prompt");
+    return -1;
+  }
+  const int n = generate_enqueued(m, prompt, n_prompt, n_steps, penalty, stop_on_eos, out_tokens,
+                                  decode_ms);
+  if (n < 0) wait_after_error(m);
   return n;
 }
 

@@ -1,5 +1,7 @@
 """Model calls that are refused or fail: what they return, and that nothing of
 them is left running or behind on the device."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -27,3 +29,47 @@ def test_step_refuses_negative_history(hip):
     same_bits(a.logits(), b.logits(), "logits")
     a.free()
     b.free()
+
+
+def test_failed_generate_leaves_nothing_running(hip):
+    """generate enqueues the prefill and then needs a longer token buffer, whose
+    allocation is refused while this thread captures another stream in global
+    mode: when the call returns its error the prefill has run to its end (the
+    state, read without waiting for the model's stream, is a plain prefill's),
+    and the model generates as before."""
+    rt = C.CDLL("libamdhip64.so")
+    vp = C.c_void_p
+    rt.hipStreamCreateWithFlags.argtypes = [C.POINTER(vp), C.c_uint]
+    rt.hipStreamBeginCapture.argtypes = [vp, C.c_int]
+    rt.hipStreamEndCapture.argtypes = [vp, C.POINTER(vp)]
+    rt.hipGraphDestroy.argtypes = [vp]
+    rt.hipStreamDestroy.argtypes = [vp]
+    blob = bh.synth_model(97, 256, 24, 8, 21, fp_sigma=0.5)
+    prompt = bh.synth_prompt(5, 97, 4001)
+    m, ref = bh.Model(blob), bh.Model(blob)
+    first, _ = m.generate(prompt, 4)
+    ref.prefill(prompt[:-1])
+    m.reset()
+    out = np.empty(5000, np.int32)  # more than the 4096 tokens a first call makes room for
+    s, g = vp(), vp()
+    assert rt.hipStreamCreateWithFlags(C.byref(s), 1) == 0
+    assert rt.hipStreamBeginCapture(s, 0) == 0
+    print("generate that fails after its prefill", flush=True)
+    rc = hip.bm_hip_model_generate(m.h, ptr(prompt), prompt.size, out.size, 1.0, 0, ptr(out), None)
+    why = bh.last_error()
+    rt.hipStreamEndCapture(s, C.byref(g))  # invalidated by the refused call
+    rt.hipGetLastError()                   # that error is this test's own
+    got = m.layer_state(m.n_layers - 1)
+    if g:
+        rt.hipGraphDestroy(g)
+    rt.hipStreamDestroy(s)
+    assert rc == -1 and "hipMalloc" in why, (rc, why)
+    want = ref.layer_state(m.n_layers - 1)
+    same_bits(got[0], want[0], "conv_state")
+    same_bits(got[1], want[1], "ssm_state")
+    assert got[2] == want[2]
+    m.reset()
+    again, _ = m.generate(prompt, 4)
+    assert list(again) == list(first)
+    m.free()
+    ref.free()
