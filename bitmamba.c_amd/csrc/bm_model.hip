@@ -1153,9 +1153,11 @@ extern "C" int bm_hip_model_config(const bm_hip_model_t* m, int which) {
 }
 
 extern "C" int bm_hip_model_reset(bm_hip_model_t* m) {
-  hipLaunchKernelGGL(bm::k_reset, dim3(512), dim3(256), 0, m->stream, m->conv_state,
-                     (size_t)m->nl * 3 * m->di, m->ssm_state, (size_t)m->nl * m->di, m->ctl);
-  MCHECK(hipGetLastError());
+  // the launch's own status: an error that an earlier call of the caller's left
+  // in this thread is not this one's
+  size_t n_conv = (size_t)m->nl * 3 * m->di, n_ssm = (size_t)m->nl * m->di;
+  void* args[] = {&m->conv_state, &n_conv, &m->ssm_state, &n_ssm, &m->ctl};
+  MCHECK(hipLaunchKernel((const void*)bm::k_reset, dim3(512), dim3(256), args, 0, m->stream));
   MCHECK(hipStreamSynchronize(m->stream));
   return 0;
 }

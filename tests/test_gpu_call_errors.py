@@ -73,3 +73,20 @@ def test_failed_generate_leaves_nothing_running(hip):
     assert list(again) == list(first)
     m.free()
     ref.free()
+
+
+def test_reset_with_an_error_pending(hip):
+    """reset does not fail for an error that the caller's own earlier HIP call
+    left in the thread."""
+    rt = C.CDLL("libamdhip64.so")
+    m = bh.Model(bh.synth_model(97, 64, 2, 4, 3, fp_sigma=0.5))
+    fresh = m.state_save()
+    m.prefill(np.array([5, 9, 3], np.int32))
+    assert m.state_save() != fresh
+    print("reset with an error pending", flush=True)
+    assert rt.hipMalloc(None, C.c_size_t(16)) != 0  # refused on the host: no pointer to fill
+    rc = hip.bm_hip_model_reset(m.h)
+    rt.hipGetLastError()
+    assert rc == 0, bh.last_error()
+    assert m.state_save() == fresh
+    m.free()
