@@ -268,7 +268,7 @@ hipError_t wait_flags(const unsigned* flags, int n, unsigned seq, hipStream_t s)
   const hipError_t e = hipStreamSynchronize(s);
   if (e != hipSuccess) return e;
   if (all_published(flags, n, seq)) return hipSuccess;
-  bm_set_error("one-launch BitLinear finished without publishing every block's completion word");
+  bm_set_error("a kernel finished without publishing every block's completion word");
   return hipErrorUnknown;
 }
 
@@ -474,12 +474,12 @@ void host_bitlinear(const float* x, int M, int n, const uint8_t* packed, int row
   const size_t obytes = (size_t)M * rows * sizeof(float);
   const size_t qbytes = (size_t)M * n;
   const size_t abytes = (size_t)M * bm::act_row_bytes(n);
-  // the results leave in one copy: [out | x_norm | int8] at 256-byte
-  // aligned offsets, the same in the device buffer and the pinned stage
+  // the results, [out | x_norm | int8] at 256-byte aligned offsets, the same in
+  // the device buffer and the pinned stage
   const size_t o_norm = bm::align_up(obytes, 256), o_q = o_norm + bm::align_up(xbytes, 256);
   const size_t iobytes = o_q + qbytes;
-  if (!ensure_dev(b.d_x, xbytes) || !ensure_dev(b.d_out, iobytes) ||
-      !ensure_dev(b.d_act, abytes) || !ensure_dev(b.d_scale, (size_t)M * 4))
+  if (!ensure_dev(b.d_out, iobytes) || !ensure_dev(b.d_act, abytes) ||
+      !ensure_dev(b.d_scale, (size_t)M * 4))
     die("scratch allocation");
   if (!ensure_pinned(b.h_stage, xbytes > iobytes ? xbytes : iobytes)) die("pinned staging");
   if (!ensure_dropin(b)) die("completion words");
@@ -489,22 +489,19 @@ void host_bitlinear(const float* x, int M, int n, const uint8_t* packed, int row
   const bool zc = o_x + xbytes <= kZeroCopyMax && ensure_mapped(b.h_zc, o_x + xbytes);
   uint8_t* hs = zc ? (uint8_t*)b.h_zc.ptr : (uint8_t*)b.h_stage.ptr;
   uint8_t* dio = zc ? (uint8_t*)b.h_zc.dev : (uint8_t*)b.d_out.ptr;
-  const float* dx = zc ? (const float*)(dio + o_x) : (const float*)b.d_x.ptr;
+  // the quantizers up to n = 8192 read x once: straight from the stage (258
+  // against 284 us per call of 256 tokens with a copy command); beyond, one
+  // that reads it three times, from a device copy
+  const bool copy_x = !zc && n > 8192;
+  if (copy_x && !ensure_dev(b.d_x, xbytes)) die("scratch allocation");
+  const float* dx = zc       ? (const float*)(dio + o_x)
+                    : copy_x ? (const float*)b.d_x.ptr
+                             : (const float*)b.h_stage.dev;
   hipStream_t s = b.stream;
   hipError_t e = hipSuccess;
   bool out_done = false;
-  if (zc) {
-    memcpy(hs + o_x, x, xbytes);
-  } else {
-    memcpy(hs, x, xbytes);
-    // the quantizers read x once: straight from the stage (258 against 284 us
-    // per call of 256 tokens with a copy command; n > 8192 takes a quantizer
-    // that reads it three times)
-    if (n <= 8192)
-      dx = (const float*)b.h_stage.dev;
-    else
-      e = hipMemcpyAsync(b.d_x.ptr, hs, xbytes, hipMemcpyHostToDevice, s);
-  }
+  memcpy(zc ? hs + o_x : hs, x, xbytes);
+  if (copy_x) e = hipMemcpyAsync(b.d_x.ptr, hs, xbytes, hipMemcpyHostToDevice, s);
   const bool generic = bm::product_needs_generic(M, cols);
   const int nblk = M == 1 && bm::rows_fit(n) ? bm::dropin_blocks(rows, n) : 0;
   if (zc && nblk > 0 && nblk <= kDropInMaxBlocks && ensure_dropin(b)) {
