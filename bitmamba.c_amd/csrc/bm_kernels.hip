@@ -1150,6 +1150,65 @@ __global__ __launch_bounds__(512) void k_gemm_few(const uint8_t* __restrict__ ac
 // Generic product for any K (K % 64 != 0 or very long rows): plain int8
 // activations, 1024-column slices then the K % 4 remainder.
 // ---------------------------------------------------------------------------
+// A wave per row and token, a packed byte and its four int8 values per lane
+// and turn: nothing to stage or to wait for, the faster way where the waves
+// fit the chip at once (generic_by_wave).
+template <int MODE>
+__global__ __launch_bounds__(256) void k_generic_wave(const int8_t* __restrict__ xq, int ldx,
+                                                      const float* __restrict__ scale_x,
+                                                      const uint8_t* __restrict__ W, int N, int K,
+                                                      float w_scale, float* __restrict__ out,
+                                                      int32_t* __restrict__ out_i32) {
+  constexpr bool I32 = MODE == 2;
+  const int m = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r >= N) return;  // whole wave leaves together
+  const int8_t* __restrict__ xr = xq + (size_t)m * ldx;
+  const uint8_t* __restrict__ row = W + (size_t)r * ((K + 3) / 4);
+  const int n_groups = K / 4;
+  const float inv = I32 ? 0.0f : inv_scale_of(scale_x[m], w_scale);
+  float o = 0.0f;
+  int tot = 0;
+  for (int g0 = 0; g0 < n_groups; g0 += 256) {
+    const int g1 = min(g0 + 256, n_groups);
+    int part = 0;
+    for (int g = g0 + lane; g < g1; g += 64) {
+      const uint32_t b = row[g];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        int w = (int)((b >> (2 * j)) & 3u) - 1;
+        w = w > 1 ? 1 : w;
+        part += w * (int)xr[4 * g + j];
+      }
+    }
+    part = wave_sum_i32(part);
+    if (I32)
+      tot += part;
+    else
+      o = __fadd_rn(o, __fmul_rn((float)part, inv));
+  }
+  if (4 * n_groups < K) {
+    int rem = 0;
+    const uint32_t b = row[n_groups];
+    for (int c = 4 * n_groups; c < K; ++c) {
+      int w = (int)((b >> (2 * (c & 3))) & 3u) - 1;
+      w = w > 1 ? 1 : w;
+      rem += w * (int)xr[c];
+    }
+    if (I32)
+      tot += rem;
+    else
+      o = __fadd_rn(o, __fmul_rn((float)rem, inv));
+  }
+  if (lane == 0) {
+    if (I32)
+      out_i32[(size_t)m * N + r] = tot;
+    else
+      out[(size_t)m * N + r] = MODE == 1 ? __fadd_rn(out[(size_t)m * N + r], o) : o;
+  }
+}
+
 // A wave takes 4 rows, 16 lanes each, and TM tokens; a lane owns 64 columns of
 // the 1024-column slice: 16 packed bytes (any alignment) and, of each token,
 // 64 int8 values that the block stages in LDS, zero past the last whole group
@@ -1157,7 +1216,9 @@ __global__ __launch_bounds__(512) void k_gemm_few(const uint8_t* __restrict__ ac
 // [token][k][lane][16 bytes], k the 16-column quarter, so that 16 lanes read
 // 256 consecutive bytes.  x.w = x.code - sum(x), v_dot4 both.
 // Latency-bound: M = 37, K = 1000, N = 1003 with its quantizer 18.7 -> 10.3 us
-// per call against a wave per row and token with byte loads (37k waves).
+// per call against k_generic_wave's 37k waves; TM the tokens there are, since a
+// wave works for all TM (N = 12000, K = 500: M = 2 3.3 us with TM = 2, 5.4 with
+// TM = 8, k_generic_wave 4.8).
 template <int MODE, int TM>
 __global__ __launch_bounds__(256) void k_generic(const int8_t* __restrict__ xq, int ldx,
                                                  const float* __restrict__ scale_x, int M,
@@ -2010,11 +2071,43 @@ static hipError_t generic_t(const int8_t* xq, int ldx, const float* scale_x, int
   return hipGetLastError();
 }
 
+// k_generic_wave up to about where its M N waves take as long as k_generic's
+// staged tiles: fewer the longer the row (k_generic's wider loads count more)
+// and the fewer the tokens (a smaller tile).  us per int32 product, by wave /
+// staged: K = 130 2.1 / 5.1 at M = 8, N = 128, 4.0 / 5.6 at 16, 1003, 10.1 / 6.7
+// at 64, 1003; K = 1000 2.5 / 5.0, 5.1 / 5.2, 14.3 / 5.6; K = 8190 8.0 / 20.6,
+// 26.4 / 20.9, 90 / 25.4.  M = 1: K = 130 2.1 / 2.5 at N = 1003, 3.4 / 3.0 at
+// 12000; K = 8190 7.9 / 5.7 at 1003.
+static bool generic_by_wave(int M, int N, int K) {
+  const size_t waves = (size_t)M * N;
+  if (M == 1) return waves <= (K < 600 ? 8192 : K < 2000 ? 3072 : 0);
+  if (M == 2) return waves <= (K < 600 ? 8192 : K < 2000 ? 4096 : 2048);
+  if (M <= 4) return waves <= (K < 600 ? 12288 : K < 2000 ? 8192 : 5120);
+  return waves <= (K < 400 ? 32768 : K < 600 ? 24576 : 16384);
+}
+
 hipError_t launch_generic(const int8_t* xq, int ldx, const float* scale_x, int M,
                           const uint8_t* packed, int N, int K, float w_scale, void* out, int mode,
                           hipStream_t s) {
   if (M <= 0) return hipSuccess;
+  if (generic_by_wave(M, N, K)) {
+    const dim3 grid((N + 3) / 4, M), block(256);
+    float* of = (float*)out;
+    int32_t* oi = (int32_t*)out;
+    if (mode == MODE_I32)
+      hipLaunchKernelGGL(k_generic_wave<2>, grid, block, 0, s, xq, ldx, scale_x, packed, N, K,
+                         w_scale, of, oi);
+    else if (mode == MODE_ACC)
+      hipLaunchKernelGGL(k_generic_wave<1>, grid, block, 0, s, xq, ldx, scale_x, packed, N, K,
+                         w_scale, of, oi);
+    else
+      hipLaunchKernelGGL(k_generic_wave<0>, grid, block, 0, s, xq, ldx, scale_x, packed, N, K,
+                         w_scale, of, oi);
+    return hipGetLastError();
+  }
   if (M == 1) return generic_t<1>(xq, ldx, scale_x, M, packed, N, K, w_scale, out, mode, s);
+  if (M == 2) return generic_t<2>(xq, ldx, scale_x, M, packed, N, K, w_scale, out, mode, s);
+  if (M <= 4) return generic_t<4>(xq, ldx, scale_x, M, packed, N, K, w_scale, out, mode, s);
   return generic_t<8>(xq, ldx, scale_x, M, packed, N, K, w_scale, out, mode, s);
 }
 
