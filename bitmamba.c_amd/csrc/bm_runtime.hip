@@ -415,9 +415,38 @@ void bitlinear_check(int n, const struct tensor* w) {
   }
 }
 
+// results from here on are copied to `out` past the CPU's caches, as one large
+// memcpy does by itself and one per slice does not: 2048 tokens, 1024 -> 4192
+// (34 MB) 2.47 -> 2.00 ms (2.35 with one copy command and one memcpy), 1280
+// tokens (21 MB) 1.30 against 1.28, 1024 (17 MB) 1.02 against 1.07
+constexpr size_t kStreamedBytes = (size_t)24 << 20;
+
 struct OutPart {
   size_t off, bytes;  // the same offset in the device buffer and the stage
 };
+
+// memcpy past the caches
+void copy_streamed(uint8_t* d, const uint8_t* s, size_t n) {
+  const size_t head = (16 - ((uintptr_t)d & 15)) & 15;
+  if (n < head + 64) {
+    memcpy(d, s, n);
+    return;
+  }
+  memcpy(d, s, head);
+  size_t i = head;
+  for (; i + 64 <= n; i += 64) {
+    const __m128i a = _mm_loadu_si128((const __m128i*)(s + i));
+    const __m128i b = _mm_loadu_si128((const __m128i*)(s + i + 16));
+    const __m128i c = _mm_loadu_si128((const __m128i*)(s + i + 32));
+    const __m128i e = _mm_loadu_si128((const __m128i*)(s + i + 48));
+    _mm_stream_si128((__m128i*)(d + i), a);
+    _mm_stream_si128((__m128i*)(d + i + 16), b);
+    _mm_stream_si128((__m128i*)(d + i + 32), c);
+    _mm_stream_si128((__m128i*)(d + i + 48), e);
+  }
+  memcpy(d + i, s + i, n - i);
+  _mm_sfence();
+}
 
 // The results of a host-pointer call: a kernel copies them to the stage (the
 // caller's `out` first, part 0) in slices, a block each, and publishes every
@@ -445,13 +474,18 @@ hipError_t results_to_host(Backend& b, const OutPart (&part)[3], uint8_t* out, u
   hipLaunchKernelGGL(bm::k_to_host, dim3(blocks), dim3(256), 0, s, hsl, dev,
                      (uint8_t*)b.h_stage.dev, (unsigned*)b.h_flag.dev, seq);
   hipError_t e = hipGetLastError();
+  const bool streamed = part[0].bytes >= kStreamedBytes;
   const unsigned* flags = (const unsigned*)b.h_flag.ptr;
   for (int k = 0; k < blocks && e == hipSuccess; ++k) {
     e = wait_flags(flags + k, 1, seq, s);
     const size_t off = (size_t)k * slice;
-    if (e == hipSuccess && off < part[0].bytes)
-      memcpy(out + off, hs + part[0].off + off,
-             part[0].bytes - off < slice ? part[0].bytes - off : slice);
+    if (e == hipSuccess && off < part[0].bytes) {
+      const size_t bytes = part[0].bytes - off < slice ? part[0].bytes - off : slice;
+      if (streamed)
+        copy_streamed(out + off, hs + part[0].off + off, bytes);
+      else
+        memcpy(out + off, hs + part[0].off + off, bytes);
+    }
   }
   return e;
 }

@@ -19,15 +19,46 @@ def inputs(M, n, rows, seed):
     return x, packed, (1.0 + 0.1 * r.standard_normal(n)).astype(np.float32)
 
 
-def host_call(hip, x, packed, g, rows, stride, norm=True, quant=True):
+def host_call(hip, x, packed, g, rows, stride, norm=True, quant=True, shift=0):
+    """The call's results; `out` starts `shift` floats into a buffer."""
     M, n = x.shape
     w, nw = bh.make_tensor(packed, rows, n, 0.02), bh.make_tensor(data=g)
-    out = np.full((M, rows), np.nan, np.float32)
+    buf = np.full(M * rows + 2 * shift, np.nan, np.float32)
+    out = buf[shift:shift + M * rows].reshape(M, rows)
     xn = np.full(n + 4, 7.0, np.float32)
     xq = np.full((M, stride), 99, np.int8)
     hip.hip_bitlinear_forward_batch(ptr(x), M, n, C.byref(w), C.byref(nw), ptr(out),
                                     ptr(xn) if norm else None, ptr(xq) if quant else None, stride)
+    assert np.isnan(buf[:shift]).all() and np.isnan(buf[M * rows + shift:]).all()
     return out, xn, xq
+
+
+def device_call(hip, x, packed, g, rows):
+    """The same product through device buffers."""
+    M, n = x.shape
+    DB = bh.DeviceBuffer
+    dx, dg, dw = DB.from_array(x), DB.from_array(g), DB.from_array(packed)
+    do, dq, ds = DB(4 * M * rows), DB(M * n), DB(4 * M)
+    da = DB(max(hip.bm_hip_act_bytes(M, n), 1))
+    bh.check(hip.bm_hip_bitlinear_dev(dx.ptr, M, n, dg.ptr, dw.ptr, rows, 0.02, 1, do.ptr, dq.ptr, n,
+                                      ds.ptr, da.ptr, None), "bitlinear")
+    hip.bm_hip_synchronize()
+    return do.download((M, rows), np.float32), dq.download((M, n), np.int8)
+
+
+@pytest.mark.parametrize("M,n,rows,shift", [(1536, 1024, 4192, 0), (1700, 1024, 4099, 1),
+                                            (6, 64, 1100000, 3)])
+def test_streamed_results(hip, M, n, rows, shift):
+    """Results beyond the caches, to outputs that start on any float."""
+    print("host batch M=%d n=%d rows=%d shift=%d" % (M, n, rows, shift), flush=True)
+    x, packed, g = inputs(M, n, rows, M + n)
+    out, xn, xq = host_call(hip, x, packed, g, rows, n + 5, shift=shift)
+    want, q = device_call(hip, x, packed, g, rows)
+    same_bits(out, want, "out")
+    np.testing.assert_array_equal(xq[:, :n], q)
+    assert (xq[:, n:] == 99).all()
+    rn, _, _, _ = native.orc_quantize_rows(x[-1:], g)
+    same_bits(xn[:n], rn[0], "x_norm")
 
 
 def test_memory_of_large_calls(hip):
