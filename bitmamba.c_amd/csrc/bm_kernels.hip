@@ -289,11 +289,14 @@ static void quantize_tok_t(const float* x, int M, int n, int x_stride, const flo
                        x_norm, xq, quant_stride, scale_x, max_out, act, act_row_bytes(n), nibbles);
 }
 
-// false beyond n = 8192
+// false beyond n = 8192, and where a chain is so short that k_quantize adds it
+// in less time than chain_wave takes for its padding (us per call, k_quantize /
+// this: n = 1 2.46 / 3.07 at one token, 6.46 / 8.76 at 4096; n = 4 2.91 / 2.85,
+// 3.57 / 3.56 at 512, 7.6 / 8.8 at 4096; n = 8 3.39 / 2.84, 8.57 / 8.79)
 static bool quantize_tok(const float* x, int M, int n, int x_stride, const float* gamma,
                          float* x_norm, int8_t* xq, int quant_stride, float* scale_x,
                          float* max_out, uint8_t* act, bool nibbles, hipStream_t s) {
-  if (n < 1 || n > 8192) return false;
+  if (n < 4 || n > 8192 || (n <= 8 && M > 512)) return false;
   auto go = [&](auto e) {
     quantize_tok_t<decltype(e)::value>(x, M, n, x_stride, gamma, x_norm, xq, quant_stride, scale_x,
                                        max_out, act, nibbles, s);

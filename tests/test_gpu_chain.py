@@ -84,6 +84,25 @@ def test_token_block_quantizer(hip, n):
         same_bits(ds.download(M, np.float32), osc, "scale")
 
 
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 7, 8])
+@pytest.mark.parametrize("M", [1, 512, 513])
+def test_narrow_rows(hip, n, M):
+    """Rows of a few values: both quantizers on either side of their rule, from
+    which the norm and the int8 rows come."""
+    print("quantize M=%d n=%d" % (M, n), flush=True)
+    r = np.random.default_rng(100 * n + M)
+    x = (r.standard_normal((M, n)) * np.exp(3.0 * r.standard_normal((M, 1)))).astype(np.float32)
+    g = (r.standard_normal(n) * 0.02).astype(np.float32)
+    dx, dg, dn, dq, ds = DB.from_array(x), DB.from_array(g), DB(4 * M * n), DB(M * n), DB(4 * M)
+    bh.check(hip.bm_hip_quantize_dev(dx.ptr, M, n, n, dg.ptr, dn.ptr, dq.ptr, n, ds.ptr, None, None),
+             "quantize")
+    hip.bm_hip_synchronize()
+    on, oq, osc, _ = native.orc_quantize_rows(x, g)
+    same_bits(dn.download((M, n), np.float32), on, "x_norm")
+    np.testing.assert_array_equal(dq.download((M, n), np.int8), oq)
+    same_bits(ds.download(M, np.float32), osc, "scale")
+
+
 def rnd_rows(n):
     return np.random.default_rng(n).standard_normal((5, n)).astype(np.float32)
 
