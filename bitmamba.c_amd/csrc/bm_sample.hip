@@ -28,6 +28,7 @@
 // like glibc's qsort (a merge sort for these sizes), keyed on the value.
 // Float-to-int bucket indices follow x86 cvttss2si (out of range -> INT_MIN).
 #include "bm_common.h"
+#include "bm_exact.h"
 #include "bm_dev.h"
 #include "bm_libm.h"
 
@@ -79,8 +80,9 @@ __device__ __forceinline__ int p_bucket(float v) {
 // scratch: probs[V], pre[kFront * seg] (also the radix sort's second
 // buffer), esum[kFront], psum[kFront], bsum[kPBuckets], pv[kFront * seg]
 // (beside pre: exp(logit - max), then the probability), bcnt[kPBuckets],
-// pmax[kFront], pcnt[kFront], hist[kBuckets].  hist is zero between calls:
-// k_samp_scale clears it, and so does k_sample after use.
+// pmax[kFront], pcnt[kFront], hist[kBuckets], scaled (whether k_samp_probs
+// could form the probabilities).  hist is zero between calls: k_samp_scale
+// clears it, and so does k_sample after use.
 struct Scratch {
   Cand* probs;
   Cand* pre;
@@ -92,6 +94,7 @@ struct Scratch {
   float* pmax;
   int* pcnt;
   int* hist;
+  int* scaled;
 };
 __host__ __device__ __forceinline__ Scratch scratch_of(void* base, int V) {
   Scratch s;
@@ -107,6 +110,7 @@ __host__ __device__ __forceinline__ Scratch scratch_of(void* base, int V) {
   s.pmax = (float*)(s.bcnt + kPBuckets);
   s.pcnt = (int*)(s.pmax + kFront);
   s.hist = s.pcnt + kFront;
+  s.scaled = s.hist + kBuckets;
   return s;
 }
 
@@ -645,11 +649,17 @@ __device__ void embed_next(int token, const StepIO& io) {
 // non-negative terms is within (n - 1) 2^-53 of the exact one, relative,
 // whatever the order; so where a sum of the same terms in another order, widened
 // by twice that and more (sum_slack), decides or rounds the same way at both
-// ends, the reference's does too.  Where it does not (about once in 10^3
-// draws, from the fp32 roundings), or where the drawn token's probability is
-// tied in the min-heap's order, draw_parallel returns false and the
-// sequential code below runs.  So does it where more than kSortMax entries
-// share the bucket that decides, and for a top_k that cuts (above 256).
+// ends, the reference's does too.  Where it does not, the sum may still be exact
+// in every order (exact_sum, bm_exact.h): sums of few terms are, and they often
+// lie on the midpoint of two floats, or on top_p itself; that is looked into
+// only then.  Where neither says (the sum over a large vocabulary close to a
+// rounding, about n 2^-26 of the draws), or where the drawn token's probability
+// is tied in the min-heap's order, draw_parallel returns false and the
+// sequential code below runs.  So does it where more than kSortMax entries share
+// the bucket that decides, and for a top_k that cuts (above 256).  Of 200 vectors
+// of spread 4 at temp = 0.8, top_p = 0.9, by the slack alone 31 went that way at
+// V = 1000, min_p = 0.05 (9 at min_p = 0) and 14 at V = 50257, min_p = 0.05; none
+// of them now.
 // V = 50257, logits of spread 4 at temp = 0.8, top_p = 0.9: 2759 us per call
 // in turn on one thread (the sum, then the heap), 48 us this way (52 with LDS
 // shuffles in the scans, 55.9 with a bitonic network for any count too).
@@ -686,18 +696,16 @@ __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlan
 __device__ __forceinline__ double sum_slack(double sum, int n) { return sum * (double)n * 0x1p-51; }
 
 // (float)sum of the reference's sum, if every sum within the slack rounds alike
-__device__ __forceinline__ bool sure_float(double sum, int n, float* f) {
-  const double d = sum_slack(sum, n);
-  *f = (float)(sum - d);
-  return uni(*f == (float)(sum + d) && *f > 0.0f && *f < __builtin_inff());
+__device__ __forceinline__ bool sure_float(double sum, double slack, float* f) {
+  *f = (float)(sum - slack);
+  return uni(*f == (float)(sum + slack) && *f > 0.0f && *f < __builtin_inff());
 }
 
-// 1 / (float)sum (src/model.c:298)
-__device__ __forceinline__ bool softmax_scale(double sum, int n, float* inv) {
-  float f;
-  const bool ok = n > 0 && sure_float(sum, n, &f);
-  *inv = ok ? cr_divf(1.0f, f) : 0.0f;
-  return ok;
+// the wave's smallest v
+__device__ __forceinline__ float wave_least(float v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
+  return lane_f32(v, 0);
 }
 
 // block-wide inclusive prefix sum; *before = the sum in front of the thread
@@ -791,9 +799,9 @@ __device__ int sort_buckets(const Scratch& sc, const int (&pc)[kListsPerWave], i
 
 __device__ __forceinline__ float key_prob(uint64_t k) { return __uint_as_float(~(uint32_t)(k >> 32)); }
 
-// first sorted entry whose running sum (from `base`) passes x -- is >= x
-// (INCL) or > x -- and whether that is sure; the running sum there in *at.
-// first: nothing comes before entry 0.  n if none passes.
+// first sorted entry whose running sum (from `base`, of larger terms) passes x
+// -- is >= x (INCL) or > x -- and whether that is sure; the running sum there in
+// *at.  first: nothing comes before entry 0.  n if none passes.
 template <bool INCL>
 __device__ int find_key(int n, double base, double x, double slack, bool first, bool* sure,
                         double* at, Smem& sm) {
@@ -832,6 +840,9 @@ __device__ int find_key(int n, double base, double x, double slack, bool first, 
   __syncthreads();
   *at = sm.dwork[0];
   *sure = uni(j < n && sm.dwork[0] > x + slack && ((first && j == 0) || sm.dwork[1] < x - slack));
+  if (!*sure && uni(j < n))  // every term so far is at least entry j's
+    *sure = uni(exact_sum(sm.dwork[0], key_prob(sm.keys[j])) &&
+                ((first && j == 0) || (INCL ? sm.dwork[1] < x : sm.dwork[1] <= x)));
   __syncthreads();
   return j;
 }
@@ -867,21 +878,46 @@ __device__ int find_bucket(const double (&s)[2], const int (&c)[2], double x, do
   return at == kPBuckets ? -1 : kPBuckets - 1 - at;
 }
 
+// the smallest listed probability that is not zero
+__device__ float least_prob(const Scratch& sc, const int (&pc)[kListsPerWave], int seg, Smem& sm) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float v = __builtin_inff();
+  for (int j = 0; j < kListsPerWave; ++j) {
+    const float* __restrict__ list = sc.pv + (size_t)(wave * kListsPerWave + j) * seg;
+    for (int i = lane; i < pc[j]; i += 64)
+      if (list[i] > 0.0f) v = fminf(v, list[i]);
+  }
+  v = wave_least(v);
+  __syncthreads();
+  if (lane == 0) sm.fred[wave] = v;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kThreads / 64; ++w) v = fminf(v, sm.fred[w]);
+  __syncthreads();
+  return v;
+}
+
 __device__ bool draw_parallel(const Scratch& sc, const int (&pc)[kListsPerWave], int seg,
                               const SampleParams& p, uint64_t& rng, int* token, Smem& sm) {
   static_assert(kFront == 64 && kPBuckets == 2 * kThreads, "lane / thread per list / buckets");
   const int lane = threadIdx.x & 63;
   const int mine = sc.pcnt[lane];
   const int n = wave_sum_i32(mine);
-  float inv, f;
-  if (!softmax_scale(wave_sum_f64(sc.esum[lane]), n, &inv)) return false;
+  float f;
+  if (!uni(*sc.scaled)) return false;
   const double ps = sc.psum[lane], total = wave_sum_f64(ps);
   const double slack = sum_slack(total, n);
+  float total_f;  // (float)total, and whether that is sure
+  bool total_sure = sure_float(total, slack, &total_f), total_exact = false;
+  if (!total_sure) {
+    total_exact = uni(exact_sum(total, least_prob(sc, pc, seg, sm)));
+    total_sure = total_exact && sure_float(total, 0.0, &total_f);
+  }
   uint64_t g = rng;
   if (p.top_p >= 1.0f && (p.top_k <= 0 || p.top_k >= n)) {
     // in index order: the list, then the entry the walk ends at
-    if (!sure_float(total, n, &f)) return false;
-    const double r = (double)__fmul_rn(rng_float(g), f);
+    if (!total_sure) return false;
+    const double r = (double)__fmul_rn(rng_float(g), total_f);
     const double incl = wave_scan_f64(ps);
     const uint64_t hit = __ballot(mine > 0 && incl > r);
     if (!hit) return false;
@@ -928,7 +964,7 @@ __device__ bool draw_parallel(const Scratch& sc, const int (&pc)[kListsPerWave],
     c[e] = sc.bcnt[b];
   }
   const double tp = (double)p.top_p;
-  double front = 0.0, kept = total;
+  double front = 0.0, kept;
   int fcnt = 0, ncut = n, held = -1, n_held = 0;  // held: the bucket(s) in sm.keys
   bool all = false, sure;
   const int bc = find_bucket<true>(s, c, tp, &front, &fcnt, sm);
@@ -941,7 +977,8 @@ __device__ bool draw_parallel(const Scratch& sc, const int (&pc)[kListsPerWave],
     return r;
   };
   if (bc < 0) {
-    if (uni(total + slack >= tp)) return false;
+    if (!total_sure || uni(total + slack >= tp && !(total_exact && total < tp))) return false;
+    f = total_f;
   } else {
     const int cnt = count_of(bc);
     all = fcnt + cnt <= kSortMax;
@@ -952,9 +989,12 @@ __device__ bool draw_parallel(const Scratch& sc, const int (&pc)[kListsPerWave],
     const int j = find_key<true>(n_held, front, tp, slack, fcnt == 0, &sure, &kept, sm);
     if (!sure) return false;
     ncut = fcnt + j + 1;
+    // every term is at least the last one
+    if (!sure_float(kept, sum_slack(kept, ncut), &f) &&
+        !(uni(exact_sum(kept, key_prob(sm.keys[j]))) && sure_float(kept, 0.0, &f)))
+      return false;
   }
   if (p.top_k > 0 && p.top_k < ncut) return false;
-  if (!sure_float(kept, n, &f)) return false;
   const double r = (double)__fmul_rn(rng_float(g), f);
   if (!all) {
     const int br = find_bucket<false>(s, c, r, &front, &fcnt, sm);
@@ -1146,18 +1186,47 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_probs(int V, void* scrat
   __shared__ double bsum[kPBuckets];
   __shared__ int bcnt[kPBuckets];
   __shared__ double wsum[kFrontThreads / 64];
+  __shared__ float wlo[kFrontThreads / 64], whi[kFrontThreads / 64];
+  static_assert(kFrontThreads == 256, "four waves");
   if (step_stopped(ctl)) return;
   const Scratch sc = scratch_of(scratch, V);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cnt = sc.pcnt[blockIdx.x];
-  const int n = wave_sum_i32(sc.pcnt[lane]);
+  const int n = uni(wave_sum_i32(sc.pcnt[lane]));
   for (int b = threadIdx.x; b < kPBuckets; b += kFrontThreads) {
     bsum[b] = 0.0;
     bcnt[b] = 0;
   }
-  float inv;
-  const bool ok = softmax_scale(wave_sum_f64(sc.esum[lane]), n, &inv);
+  // 1 / (float)sum (src/model.c:298)
+  const double esum = wave_sum_f64(sc.esum[lane]);
+  float f;
+  bool ok = n > 0 && sure_float(esum, sum_slack(esum, n), &f);
+  if (n > 0 && !ok) {
+    // exact?  The smallest numerator from the smallest candidate, halved: expf
+    // is monotone but for its last bit
+    float lo = __builtin_inff(), hi = -__builtin_inff();
+    for (int l = 0; l < kFront; ++l) {
+      const Cand* __restrict__ list = sc.pre + (size_t)l * front_seg(V);
+      for (int i = threadIdx.x; i < sc.pcnt[l]; i += kFrontThreads) {
+        lo = fminf(lo, list[i].val);
+        hi = fmaxf(hi, list[i].val);
+      }
+    }
+    lo = wave_least(lo);
+    hi = -wave_least(-hi);
+    if (lane == 0) {
+      wlo[wave] = lo;
+      whi[wave] = hi;
+    }
+    __syncthreads();
+    lo = fminf(fminf(wlo[0], wlo[1]), fminf(wlo[2], wlo[3]));
+    hi = fmaxf(fmaxf(whi[0], whi[1]), fmaxf(whi[2], whi[3]));
+    const float least = 0.5f * libm::expf_glibc(__fsub_rn(lo, hi));
+    ok = uni(exact_sum(esum, least)) && sure_float(esum, 0.0, &f);
+  }
+  const float inv = ok ? cr_divf(1.0f, f) : 0.0f;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *sc.scaled = ok;
   __syncthreads();
-  if (!ok) return;  // k_sample finds the same and takes the sequential path
+  if (!ok) return;  // k_sample takes the sequential path
   float* pv = sc.pv + (size_t)blockIdx.x * front_seg(V);
   double sum = 0.0;
   for (int i = threadIdx.x; i < cnt; i += kFrontThreads) {
@@ -1364,7 +1433,7 @@ size_t sample_scratch_bytes(int V) {
   const size_t lists = (size_t)kFront * front_seg(V);
   // + 32: the two alignments of scratch_of
   return ((size_t)V + lists) * sizeof(Cand) + (2 * kFront + kPBuckets) * sizeof(double) +
-         (lists + kPBuckets + 2 * kFront + kBuckets) * sizeof(int) + 32;
+         (lists + kPBuckets + 2 * kFront + kBuckets + 1) * sizeof(int) + 32;
 }
 
 // pmax/npart: the maxima of logits already scaled by 1/temp (the LM head's
