@@ -205,9 +205,12 @@ __host__ __device__ __forceinline__ int effective_k(int top_k) {
 
 // Without top-k: whether draw_parallel is tried.  Not where min_p alone cuts
 // (top_p >= 1): it leaves few candidates, which one thread walks in 16 us per
-// call, 19 with the probabilities' launch and the buckets.
-__host__ __device__ __forceinline__ bool tries_parallel(const SampleParams& p) {
-  return p.top_p < 1.0f || !(p.min_p > 0.0f);
+// call, 19 with the probabilities' launch and the buckets; for the same reason
+// not for small vocabularies at top_p >= 1 (V = 64: 17.3 us, 18.9 tried; 256: 30.7,
+// 19.0); and not where a top_k above 256 alone cuts, which only the full sort
+// decides.
+__host__ __device__ __forceinline__ bool tries_parallel(const SampleParams& p, int V) {
+  return p.top_p < 1.0f || (!(p.min_p > 0.0f) && V >= 96 && (p.top_k <= 0 || p.top_k >= V));
 }
 
 __device__ __forceinline__ float bucket_scale_of() {
@@ -1465,7 +1468,7 @@ hipError_t launch_sample(float* logits, int V, float temp, float min_p, float to
                        npart, gate);
     hipLaunchKernelGGL((k_sample<true, false>), one, all, 0, s, logits, V, p, rng_state, scratch,
                        pmax, npart, io);
-  } else if (tries_parallel(p)) {
+  } else if (tries_parallel(p, V)) {
     hipLaunchKernelGGL((k_samp_hist<false, true>), front, ft, 0, s, logits, V, p, scratch, pmax,
                        npart, gate);
     hipLaunchKernelGGL(k_samp_probs, front, ft, 0, s, V, scratch, gate);

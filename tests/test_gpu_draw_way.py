@@ -26,14 +26,16 @@ class Sampler:
 
     def draw(self, logits, temp, min_p, top_p, top_k, rng):
         """(token, generator state, True for the sequential way); the token, the
-        state and the scaled logits are the oracle's."""
+        state and the scaled logits are the oracle's.  self.tried: whether the
+        parallel draw's sums were formed at all."""
         V, hip = self.V, self.hip
         buf = np.zeros(self.pad, np.float32)
         buf[:V] = logits
         for b, a in ((self.dl, buf), (self.dr, np.array([rng], np.uint64))):
             bh.check(hip.bm_hip_memcpy_h2d(b.ptr, ptr(a), a.nbytes), "upload")
         n_cand = (V + 1) // 2 * 2 + 64 * self.seg
-        bh.check(hip.bm_hip_memset(self.ws.ptr, 0xA5, 8 * n_cand), "pattern")
+        sums = 8 * (2 * 64 + 2048) + 4 * 64 * self.seg  # after the candidates: sums and terms
+        bh.check(hip.bm_hip_memset(self.ws.ptr, 0xA5, 8 * n_cand + sums), "pattern")
         bh.check(hip.bm_hip_sample_advanced(self.dl.ptr, V, temp, min_p, top_p, top_k, self.dr.ptr,
                                             self.ws.ptr, self.dt.ptr, None), "sample_advanced")
         hip.bm_hip_synchronize()
@@ -44,7 +46,9 @@ class Sampler:
         want = native.oracle().orc_sample(ptr(ref), V, temp, min_p, top_p, top_k, C.byref(st))
         same_bits(scaled, ref, "scaled logits")
         assert (tok, state) == (want, st.value)
-        got = self.ws.download(8 * n_cand, np.uint8).view(CAND)
+        got = self.ws.download(8 * n_cand + sums, np.uint8)
+        self.tried = bool((got[8 * n_cand:] != 0xA5).any())
+        got = got[:8 * n_cand].view(CAND)
         cand, pre = got[:(V + 1) // 2 * 2], got[(V + 1) // 2 * 2:]
         touched = (cand.view(np.uint64) != 0xA5A5A5A5A5A5A5A5).any()
         pre = pre[pre.view(np.uint64) != 0xA5A5A5A5A5A5A5A5]
@@ -101,3 +105,31 @@ def test_sums_at_midpoints(hip):
         for top_p in (0.5, 0.9):
             _, _, seq = s.draw(logits, 1.0, 0.0, top_p, 0, int(r.integers(1, 2 ** 62)))
             assert not seq
+
+
+@pytest.mark.parametrize("V,min_p,top_p,top_k,tried", [
+    (95, 0.0, 1.0, 0, False), (96, 0.0, 1.0, 0, True), (5, 0.0, 0.9, 0, True),
+    (300, 0.0, 1.0, 299, False), (300, 0.0, 1.0, 300, True), (300, 0.0, 1.0, 301, True),
+    (5000, 0.0, 1.0, 257, False), (5000, 0.0, 0.9, 257, True), (5000, 0.05, 1.0, 0, False),
+    (1, 0.0, 1.0, 0, False)])
+def test_when_it_is_tried(hip, V, min_p, top_p, top_k, tried):
+    """Calls that only the sequential way can decide, or decides sooner, do not
+    pay for the parallel draw's sums."""
+    s = Sampler(hip, V)
+    r = np.random.default_rng(V + top_k)
+    for i in range(4):
+        print("V=%d min_p=%g top_p=%g top_k=%d" % (V, min_p, top_p, top_k), flush=True)
+        s.draw((r.standard_normal(V) * 2.0).astype(np.float32), 0.9, min_p, top_p, top_k, 31 * i + 7)
+        assert s.tried == tried
+
+
+def test_positive_infinity(hip):
+    """One infinite logit: every probability is NaN or 0 in the reference, and the
+    draw goes the sequential way."""
+    V = 1000
+    s = Sampler(hip, V)
+    logits = np.random.default_rng(5).standard_normal(V).astype(np.float32)
+    logits[417] = np.inf
+    print("+inf", flush=True)
+    _, _, seq = s.draw(logits, 1.0, 0.0, 1.0, 0, 12345)
+    assert seq
