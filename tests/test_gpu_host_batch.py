@@ -46,19 +46,57 @@ def device_call(hip, x, packed, g, rows):
     return do.download((M, rows), np.float32), dq.download((M, n), np.int8)
 
 
+def check(hip, M, n, rows, stride, norm=True, quant=True, shift=0, tokens=()):
+    """The host call against the device product, the oracle's norm of the last
+    token (all that x_norm keeps), and the oracle's rows of `tokens`."""
+    print("host batch M=%d n=%d rows=%d stride=%d norm=%d quant=%d" % (M, n, rows, stride, norm,
+                                                                       quant), flush=True)
+    x, packed, g = inputs(M, n, rows, M + n + rows)
+    out, xn, xq = host_call(hip, x, packed, g, rows, stride, norm, quant, shift)
+    want, q = device_call(hip, x, packed, g, rows)
+    same_bits(out, want, "out")
+    if norm:
+        rn, _, _, _ = native.orc_quantize_rows(x[-1:], g)
+        same_bits(xn[:n], rn[0], "x_norm")
+    assert (xn[n if norm else 0:] == 7.0).all()
+    if quant:
+        np.testing.assert_array_equal(xq[:, :n], q)
+    assert (xq[:, n if quant else 0:] == 99).all()
+    for m in tokens:
+        ref, _, rq = native.orc_bitlinear(x[m:m + 1], packed, rows, n, 0.02, g)
+        same_bits(out[m], ref[0], "out[%d]" % m)
+        if quant:
+            np.testing.assert_array_equal(xq[m, :n], rq[0])
+
+
+@pytest.mark.parametrize("norm,quant", [(True, True), (False, True), (True, False), (False, False)])
+@pytest.mark.parametrize("M,n,rows,stride", [
+    (256, 1024, 4192, 1024),    # slices of all three parts
+    (130, 1003, 517, 1010),     # the last x_norm on no 16 bytes: bytes; the generic product
+    (63, 1025, 1, 1025),        # results of a few bytes per token
+    (40, 8256, 300, 8300),      # x from a device copy
+    (70, 2048, 1024, 2048)])
+def test_large_calls(hip, M, n, rows, stride, norm, quant):
+    check(hip, M, n, rows, stride, norm, quant, tokens=(0, M // 2, M - 1))
+
+
+def test_large_then_small(hip):
+    """Calls of falling and rising size on one stage and one set of words."""
+    for M, n, rows in ((512, 1024, 4192), (33, 2048, 1024), (3, 1024, 300), (512, 1024, 4192),
+                       (90, 1088, 700), (1, 2048, 70001), (40, 8256, 300), (256, 1024, 512)):
+        check(hip, M, n, rows, n + 16, tokens=(0, M - 1))
+
+
+def test_more_slices_than_words(hip):
+    """147 MB of results: slices of 128 KiB."""
+    check(hip, 9000, 64, 4096, 64, tokens=(0, 4500, 8999))
+
+
 @pytest.mark.parametrize("M,n,rows,shift", [(1536, 1024, 4192, 0), (1700, 1024, 4099, 1),
                                             (6, 64, 1100000, 3)])
 def test_streamed_results(hip, M, n, rows, shift):
     """Results beyond the caches, to outputs that start on any float."""
-    print("host batch M=%d n=%d rows=%d shift=%d" % (M, n, rows, shift), flush=True)
-    x, packed, g = inputs(M, n, rows, M + n)
-    out, xn, xq = host_call(hip, x, packed, g, rows, n + 5, shift=shift)
-    want, q = device_call(hip, x, packed, g, rows)
-    same_bits(out, want, "out")
-    np.testing.assert_array_equal(xq[:, :n], q)
-    assert (xq[:, n:] == 99).all()
-    rn, _, _, _ = native.orc_quantize_rows(x[-1:], g)
-    same_bits(xn[:n], rn[0], "x_norm")
+    check(hip, M, n, rows, n + 5, shift=shift)
 
 
 def test_memory_of_large_calls(hip):
