@@ -250,8 +250,8 @@ def test_odd_shapes_vs_oracle(hip, vocab, d_model, n_heads, penalty, sampler):
 
 
 # GEMM tiles of the 1B width: 300 tokens 64x128, 1220 in_proj 128x128, 2100
-# 128x256 (three SSM chunks); 255M width, 1030 tokens: in_proj 128x256,
-# out_proj 64x128, two SSM chunks; d_model 320: out_proj (K=640 -> N=320)
+# 128x256; 255M width, 1030 tokens: in_proj 128x256, out_proj 64x128; head
+# dims of 64, whose SSM is one kernel for the whole prompt; d_model 320: out_proj (K=640 -> N=320)
 # in 64x128 tiles with 128-deep stages, its residual add over ragged last
 # row and column tiles; 1600 tokens: out_proj in 64x256 tiles
 @pytest.mark.parametrize("d_model,n_heads,n_tokens", [(1024, 32, 1030), (2048, 64, 300),
@@ -260,9 +260,9 @@ def test_odd_shapes_vs_oracle(hip, vocab, d_model, n_heads, penalty, sampler):
 def test_wide_model_long_prefill_vs_oracle(hip, d_model, n_heads, n_tokens):
     """Long prompts at the 255M and 1B widths (two layers, 2000-token
     vocabulary): the batched path with MFMA GEMM tiles, the quantize kernels
-    at K = 1024 .. 4096 and, at 1030 tokens, two chunks of the three-phase
-    SSM with 64-channel heads.  Every state value and the next step's logits
-    bit-exact against the oracle's token-serial prefill."""
+    at K = 1024 .. 4096 and the one-kernel SSM with 64-channel heads over 5 to
+    33 of its tiles.  Every state value and the next step's logits bit-exact
+    against the oracle's token-serial prefill."""
     note("wide model long prefill d_model=%d tokens=%d" % (d_model, n_tokens))
     blob = bh.synth_model(2000, d_model, 2, n_heads, 91 + d_model, bh.SYNTH_UNIFORM)
     prompt = bh.synth_prompt(91, 2000, n_tokens + 1)
@@ -291,10 +291,9 @@ def test_wide_model_long_prefill_vs_oracle(hip, d_model, n_heads, n_tokens):
 
 def test_prefill_lengths_vs_oracle(hip):
     """Prefill in one call and in several (the conv ring and the state carry
-    over), with 1 to 2050 tokens (several 1024-token chunks of the
-    three-phase SSM, counts that are not whole 4-token quads): every layer's
-    state and the next step's logits bit-exact against the oracle's
-    token-serial prefill."""
+    over), with 1 to 2050 tokens (1 to 33 tiles of the one-kernel SSM, counts
+    that fill no tile): every layer's state and the next step's logits
+    bit-exact against the oracle's token-serial prefill."""
     g = gold("tiny")
     blob, _, _ = model_image(g)
     c = g["config"]
