@@ -843,7 +843,7 @@ __device__ int find_key(int n, double base, double x, double slack, bool first, 
   __syncthreads();
   *at = sm.dwork[0];
   *sure = uni(j < n && sm.dwork[0] > x + slack && ((first && j == 0) || sm.dwork[1] < x - slack));
-  if (!*sure && uni(j < n))  // every term so far is at least entry j's
+  if (__builtin_expect(!*sure && uni(j < n), 0))  // every term so far is at least entry j's
     *sure = uni(exact_sum(sm.dwork[0], key_prob(sm.keys[j])) &&
                 ((first && j == 0) || (INCL ? sm.dwork[1] < x : sm.dwork[1] <= x)));
   __syncthreads();
@@ -907,20 +907,20 @@ __device__ bool draw_parallel(const Scratch& sc, const int (&pc)[kListsPerWave],
   const int mine = sc.pcnt[lane];
   const int n = wave_sum_i32(mine);
   float f;
-  if (!uni(*sc.scaled)) return false;
-  const double ps = sc.psum[lane], total = wave_sum_f64(ps);
+  const int scaled = *sc.scaled;
+  const double ps = sc.psum[lane];
+  if (!uni(scaled)) return false;
+  const double total = wave_sum_f64(ps);
   const double slack = sum_slack(total, n);
-  float total_f;  // (float)total, and whether that is sure
-  bool total_sure = sure_float(total, slack, &total_f), total_exact = false;
-  if (!total_sure) {
-    total_exact = uni(exact_sum(total, least_prob(sc, pc, seg, sm)));
-    total_sure = total_exact && sure_float(total, 0.0, &total_f);
-  }
+  auto total_sure = [&](float* v) {  // (float)total
+    return sure_float(total, slack, v) ||
+           (uni(exact_sum(total, least_prob(sc, pc, seg, sm))) && sure_float(total, 0.0, v));
+  };
   uint64_t g = rng;
   if (p.top_p >= 1.0f && (p.top_k <= 0 || p.top_k >= n)) {
     // in index order: the list, then the entry the walk ends at
-    if (!total_sure) return false;
-    const double r = (double)__fmul_rn(rng_float(g), total_f);
+    if (!total_sure(&f)) return false;
+    const double r = (double)__fmul_rn(rng_float(g), f);
     const double incl = wave_scan_f64(ps);
     const uint64_t hit = __ballot(mine > 0 && incl > r);
     if (!hit) return false;
@@ -980,8 +980,7 @@ __device__ bool draw_parallel(const Scratch& sc, const int (&pc)[kListsPerWave],
     return r;
   };
   if (bc < 0) {
-    if (!total_sure || uni(total + slack >= tp && !(total_exact && total < tp))) return false;
-    f = total_f;
+    if (uni(total + slack >= tp) || !total_sure(&f)) return false;
   } else {
     const int cnt = count_of(bc);
     all = fcnt + cnt <= kSortMax;
@@ -1194,16 +1193,16 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_probs(int V, void* scrat
   if (step_stopped(ctl)) return;
   const Scratch sc = scratch_of(scratch, V);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cnt = sc.pcnt[blockIdx.x];
+  // 1 / (float)sum (src/model.c:298)
   const int n = uni(wave_sum_i32(sc.pcnt[lane]));
+  const double esum = wave_sum_f64(sc.esum[lane]);
   for (int b = threadIdx.x; b < kPBuckets; b += kFrontThreads) {
     bsum[b] = 0.0;
     bcnt[b] = 0;
   }
-  // 1 / (float)sum (src/model.c:298)
-  const double esum = wave_sum_f64(sc.esum[lane]);
   float f;
   bool ok = n > 0 && sure_float(esum, sum_slack(esum, n), &f);
-  if (n > 0 && !ok) {
+  if (__builtin_expect(n > 0 && !ok, 0)) {
     // exact?  The smallest numerator from the smallest candidate, halved: expf
     // is monotone but for its last bit
     float lo = __builtin_inff(), hi = -__builtin_inff();
