@@ -64,7 +64,7 @@ __device__ __forceinline__ void stage_load(float4 (&st)[C], const float* __restr
 }
 
 struct Lds {
-  float* sq;      // [4][stride] squares, chain-major (chain_wave's layout)
+  float* sq;      // [4][stride] squares, chain-major (chain_wave's layout, or chain_regs')
   uint32_t* nib;  // [K/4] split-nibble activations
   int8_t* q8;     // [K] int8 activations
   int* slices;    // [S] sum of int8 per 1024-column slice
@@ -211,9 +211,9 @@ __device__ float pro_quant(const float4 (&xv)[C], const float4 (&gv)[C], float r
 // 4G consecutive columns (float4s G*t .. G*t+G-1) in registers for the whole
 // prologue, so all four waves share the scaling and packing work whatever K
 // is; the R = 4/G threads of a 16-column group sit in consecutive lanes.
-// The squares go through LDS once to reach the chain layout, wave 0 runs the
-// chains, and the int8 values are packed straight from registers.  Returns
-// scale_x.
+// The squares go through LDS once to reach the chain layout, wave j runs chain
+// j (wave 0 all four where `ONE` says so, below), and the int8 values are packed
+// straight from registers.  Returns scale_x.
 //   PRENORM: x first becomes (x * rms(x)) * g_pre (the final norm).
 // ---------------------------------------------------------------------------
 template <int G, bool ONE>

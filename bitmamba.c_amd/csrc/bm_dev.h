@@ -227,8 +227,8 @@ __device__ __forceinline__ float chain_regs(const float* __restrict__ sq, int st
 // of normal squares takes ~1450 / 2200 cycles at 512 / 1024 elements (K =
 // 2048 / 4096), against ~2500 / 5000 for one lane adding in turn; at 256 (K =
 // 1024) both take ~1250, and chain_regs stays.  Per launch of the 1B decode:
-// out_proj 5.78 -> 4.57 us, in_proj 5.61 -> 5.34; the greedy step 0.2895 ->
-// 0.260 ms.
+// out_proj 5.78 -> 4.57 us, in_proj 5.61 -> 5.34; the greedy step, with the
+// libm tables in LDS, 0.289 -> 0.265 ms.
 // ---------------------------------------------------------------------------
 template <int CTRL, int ROWS = 0xf>
 __device__ __forceinline__ int dpp_or0(int v) {  // lanes without a source get 0

@@ -274,7 +274,8 @@ __global__ __launch_bounds__(256) void k_ssm_out(const float* __restrict__ pre,
 // registers of the thread that needs it two iterations later, so of the
 // three-phase version's planes nothing goes through memory.  A tile's inputs
 // are loaded one iteration ahead; loads and stores are unconditional (through
-// bounds-checked buffers) so that a wait covers only what it needs.  Tokens past n carry decay 1 and xa * B * dt = -0.
+// bounds-checked buffers) so that a wait covers only what it needs.  Tokens
+// past n carry decay 1 and xa * B * dt = -0.
 // What bounds it: ~1.1 us per tile, the task waves' dependent fp64 chains (two
 // silu deep, ~220 instructions per wave and tile, two task waves per SIMD).
 // Tried without gain: task waves moved off the SIMDs of waves 0 and 1 (12
@@ -283,8 +284,8 @@ __global__ __launch_bounds__(256) void k_ssm_out(const float* __restrict__ pre,
 // 22 us (27.3 with plain loads whose row or ring address is chosen per lane,
 // a branch around each; 23.9 with the recurrence reading each quad as it
 // comes) against 17.6 + 13.9 + 13.9 us for the three kernels, whose planes
-// were ~130 MB of traffic.  The prefill of 1024 tokens 2.46 -> 1.77 ms, of 8
-// tokens 0.92 -> 0.65 ms, with the quantizers' change in both.
+// were ~130 MB of traffic.  The prefill of 1024 tokens 2.59 -> 1.96 ms, of 8
+// tokens 0.92 -> 0.67 ms, with the quantizers' change in both.
 constexpr int kFc = 16, kFt = 64, kFwaves = 10;  // channels, tokens per tile, waves
 
 __global__ __launch_bounds__(64 * kFwaves) void k_ssm_fused(

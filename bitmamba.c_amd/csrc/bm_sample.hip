@@ -12,8 +12,8 @@
 //                 lowest threshold the extraction can use (the histogram's
 //                 last bucket, or the min_p threshold), a superset of the
 //                 candidates.
-//   k_samp_probs  (no top-k, see tries_parallel) the probabilities, and per value bucket their
-//                 count and sum.
+//   k_samp_probs  (no top-k, see tries_parallel) the probabilities, and per
+//                 value bucket their count and sum.
 // k_sample then runs the rest on one 1024-thread block: the cutoff bucket,
 // the candidates filtered from the pre-candidate lists in order, selection,
 // softmax, sorting and the draw, the step bookkeeping and the next token's
@@ -1026,8 +1026,8 @@ __device__ bool draw_parallel(const Scratch& sc, const int (&pc)[kListsPerWave],
 
 // Front pass 1: logits[i] *= 1/temp over the block's segment and the
 // segment's max under `x > m` from -1e30f (src/model.c:160-166).  Block 0
-// also clears the histogram and the block counter of pass 2.  (The LM head
-// can do this pass itself, with its own blocks' maxima.)
+// also clears the histogram.  (The LM head can do this pass itself, with its
+// own blocks' maxima.)
 __global__ __launch_bounds__(kFrontThreads) void k_samp_scale(float* __restrict__ logits, int V,
                                                               float temp, void* scratch,
                                                               const int* ctl) {
@@ -1070,11 +1070,13 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_scale(float* __restrict_
 }
 
 // Front pass 2, kFront blocks: with the global max (of the npart partial
-// maxima in pmax), each block -- without top-k: also exp(logit - max) of its
-// candidates into pv and their sum; with top-k: -- adds its segment's counts to the 128-bucket
-// histogram over logits >= the min_p threshold (src/model.c:180-194) and
-// writes its pre-candidates: (i, logits[i]) with logits[i] >= the lowest
-// extraction threshold, in index order, to pre[block * seg ..].
+// maxima in pmax), each block writes its segment's pre-candidates: (i,
+// logits[i]) with logits[i] >= the lowest extraction threshold, in index
+// order, to pre[block * seg ..].
+// TOPK: it also adds the segment's counts to the 128-bucket histogram over
+// logits >= the min_p threshold (src/model.c:180-194).  PAR (tries_parallel):
+// it also writes exp(logit - max) of the candidates to pv and their sum to
+// esum.  Neither (min_p alone, say): the pre-candidates only.
 template <bool TOPK, bool PAR>
 __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __restrict__ logits,
                                                              int V, SampleParams p,
@@ -1181,7 +1183,7 @@ __global__ __launch_bounds__(kFrontThreads) void k_samp_hist(const float* __rest
   if (threadIdx.x == 0) sc.pcnt[blockIdx.x] = off;
 }
 
-// Front pass 3 (no top-k), kFront blocks: the probabilities pv * 1/sum, their
+// Front pass 3 (PAR), kFront blocks: the probabilities pv * 1/sum, their
 // sum per block, and the count and sum of each value bucket over all blocks.
 __global__ __launch_bounds__(kFrontThreads) void k_samp_probs(int V, void* scratch,
                                                               const int* ctl) {
@@ -1347,57 +1349,57 @@ __global__ __launch_bounds__(1024) void k_sample(const float* __restrict__ logit
     bool drawn = false;
     if constexpr (PAR) drawn = draw_parallel(sc, pc, seg, p, rng, &token, sm);
     if (!drawn) {
-    // no top-k: every candidate over the min_p threshold (src/model.c:278-300)
-    Cand* probs2 = sc.pre;  // free once the candidates are gathered
-    int n = gather(sc, pc, seg, min_p_thresh, sc.probs, &probs, sm);
-    if (n == 0) {
-      token = argmax_scan(logits, V, logits[0], sm);
-    } else {
-      for (int i = threadIdx.x; i < n; i += kThreads)
-        probs[i].val = libm::expf_glibc(__fsub_rn(probs[i].val, max_logit));
-      __syncthreads();
-      const double sum_exp = ordered_sum(probs, n, sm);
-      if (threadIdx.x == 0) sm.fwork[1] = cr_divf(1.0f, (float)sum_exp);
-      __syncthreads();
-      const float inv_sum = sm.fwork[1];
-      for (int i = threadIdx.x; i < n; i += kThreads) probs[i].val = __fmul_rn(probs[i].val, inv_sum);
-      __syncthreads();
-      bool done = false;
-      if (p.top_p >= 1.0f && (p.top_k <= 0 || p.top_k >= n)) {  // src/model.c:306-307
-        // order-independent: the candidates stay in index order
-        token = filter_and_sample(probs, n, p.top_p, p.top_k, rng, sm);
-        done = true;
-      }
-      if (!done && p.top_p < 1.0f && n > kPartial) {  // src/model.c:313-343
-        heap_select(probs, n, kPartial, sm.sel, sm);
-        sort_small(sm.sel, sm.sorted, kPartial);
-        if (threadIdx.x == 0) {
-          double cs = 0.0;
-          int hit = 0;
-          for (int i = 0; i < kPartial; ++i) {
-            cs += (double)sm.sorted[i].val;
-            if (cs >= (double)p.top_p) {
-              hit = 1;
-              break;
+      // no top-k: every candidate over the min_p threshold (src/model.c:278-300)
+      Cand* probs2 = sc.pre;  // free once the candidates are gathered
+      int n = gather(sc, pc, seg, min_p_thresh, sc.probs, &probs, sm);
+      if (n == 0) {
+        token = argmax_scan(logits, V, logits[0], sm);
+      } else {
+        for (int i = threadIdx.x; i < n; i += kThreads)
+          probs[i].val = libm::expf_glibc(__fsub_rn(probs[i].val, max_logit));
+        __syncthreads();
+        const double sum_exp = ordered_sum(probs, n, sm);
+        if (threadIdx.x == 0) sm.fwork[1] = cr_divf(1.0f, (float)sum_exp);
+        __syncthreads();
+        const float inv_sum = sm.fwork[1];
+        for (int i = threadIdx.x; i < n; i += kThreads) probs[i].val = __fmul_rn(probs[i].val, inv_sum);
+        __syncthreads();
+        bool done = false;
+        if (p.top_p >= 1.0f && (p.top_k <= 0 || p.top_k >= n)) {  // src/model.c:306-307
+          // order-independent: the candidates stay in index order
+          token = filter_and_sample(probs, n, p.top_p, p.top_k, rng, sm);
+          done = true;
+        }
+        if (!done && p.top_p < 1.0f && n > kPartial) {  // src/model.c:313-343
+          heap_select(probs, n, kPartial, sm.sel, sm);
+          sort_small(sm.sel, sm.sorted, kPartial);
+          if (threadIdx.x == 0) {
+            double cs = 0.0;
+            int hit = 0;
+            for (int i = 0; i < kPartial; ++i) {
+              cs += (double)sm.sorted[i].val;
+              if (cs >= (double)p.top_p) {
+                hit = 1;
+                break;
+              }
             }
+            sm.iwork[1] = hit;
           }
-          sm.iwork[1] = hit;
-        }
-        __syncthreads();
-        done = sm.iwork[1] != 0;
-        __syncthreads();
-        if (done) {
-          // sm.sorted is read through the staging buffer
-          for (int i = threadIdx.x; i < kPartial; i += kThreads) sm.sel[i] = sm.sorted[i];
           __syncthreads();
-          token = filter_and_sample(sm.sel, kPartial, p.top_p, p.top_k, rng, sm);
+          done = sm.iwork[1] != 0;
+          __syncthreads();
+          if (done) {
+            // sm.sorted is read through the staging buffer
+            for (int i = threadIdx.x; i < kPartial; i += kThreads) sm.sel[i] = sm.sorted[i];
+            __syncthreads();
+            token = filter_and_sample(sm.sel, kPartial, p.top_p, p.top_k, rng, sm);
+          }
+        }
+        if (!done) {  // full sort (src/model.c:345-347)
+          sort_large(probs, probs2, n, sm);
+          token = filter_and_sample(probs, n, p.top_p, p.top_k, rng, sm);
         }
       }
-      if (!done) {  // full sort (src/model.c:345-347)
-        sort_large(probs, probs2, n, sm);
-        token = filter_and_sample(probs, n, p.top_p, p.top_k, rng, sm);
-      }
-    }
     }
   }
 

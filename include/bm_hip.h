@@ -394,8 +394,10 @@ int bm_hip_model_set_sampler(bm_hip_model_t *m,
  * logits[vocab] (device memory, 16-byte aligned; scaled in place by 1/temp
  * as the reference leaves them), advancing the XorShift64* state *rng
  * (device memory, src/utils.c:117-140); temp < 0.05 is the greedy branch.
- * workspace: bm_hip_sample_workspace_bytes(vocab) bytes of device memory
- * (the reference's probs buffer, twice).  The token goes to token_out[0]
+ * workspace: bm_hip_sample_workspace_bytes(vocab) bytes of device memory, on
+ * any alignment and with any contents (the reference's probs buffer, candidate
+ * lists and partial sums: no multiple of the vocabulary, ask the function).
+ * The token goes to token_out[0]
  * (device memory); enqueued on `stream`, no synchronization.  0, or -1 for
  * vocab outside 1..256000, misaligned logits or a null pointer. */
 size_t bm_hip_sample_workspace_bytes(int vocab);
