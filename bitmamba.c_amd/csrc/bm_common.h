@@ -72,9 +72,11 @@ hipError_t launch_small_i8(const int8_t *xq, int M, int ldx, int K, const uint8_
                            bool canonical, int32_t *out, hipStream_t s);
 bool product_needs_generic(int M, int K);
 bool product_reads_nibbles(int M, int N, int K);
+// x_on_host: xq lies in mapped host memory
 hipError_t launch_generic(const int8_t *xq, int ldx, const float *scale_x,
                           int M, const uint8_t *packed, int N, int K,
-                          float w_scale, void *out, int mode, hipStream_t s);
+                          float w_scale, void *out, int mode, hipStream_t s,
+                          bool x_on_host = false);
 hipError_t launch_rms_norm(const float *x, int n, const float *gamma,
                            float *out, float *max_out, hipStream_t s);
 hipError_t launch_canonicalize(uint8_t *p, size_t bytes, hipStream_t s);

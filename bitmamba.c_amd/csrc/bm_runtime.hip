@@ -554,7 +554,7 @@ void host_bitlinear(const float* x, int M, int n, const uint8_t* packed, int row
     if (e == hipSuccess) {
       if (generic)
         e = bm::launch_generic((const int8_t*)(dio + o_q), n, (const float*)b.d_scale.ptr, M, dW,
-                               rows, cols, w_scale, dio, bm::MODE_STORE, s);
+                               rows, cols, w_scale, dio, bm::MODE_STORE, s, zc);
       else
         e = bm::launch_product((const uint8_t*)b.d_act.ptr, (const float*)b.d_scale.ptr, M, dW,
                                rows, cols, w_scale, true, dio, bm::MODE_STORE, s);

@@ -1,6 +1,6 @@
-"""The host-pointer batch call above the zero-copy size: results that leave in
+"""The host-pointer batch call: above the zero-copy size, results that leave in
 published slices, x read from the pinned stage or copied, and the memory that
-the call holds."""
+the call holds; below it, odd widths."""
 import ctypes as C
 
 import numpy as np
@@ -78,6 +78,14 @@ def check(hip, M, n, rows, stride, norm=True, quant=True, shift=0, tokens=()):
     (70, 2048, 1024, 2048)])
 def test_large_calls(hip, M, n, rows, stride, norm, quant):
     check(hip, M, n, rows, stride, norm, quant, tokens=(0, M // 2, M - 1))
+
+
+@pytest.mark.parametrize("M", [1, 2, 3])
+@pytest.mark.parametrize("n,rows", [(130, 17), (1003, 1003), (2050, 64)])
+def test_small_odd_widths(hip, M, n, rows):
+    """Zero-copy calls at widths off 64: the product reads its int8 rows from the
+    mapped memory, one or two of them staged, more by a wave each."""
+    check(hip, M, n, rows, n + 2, tokens=range(M))
 
 
 def test_large_then_small(hip):
