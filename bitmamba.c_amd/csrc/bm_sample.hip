@@ -907,15 +907,14 @@ __device__ bool draw_parallel(const Scratch& sc, const int (&pc)[kListsPerWave],
   const int mine = sc.pcnt[lane];
   const int n = wave_sum_i32(mine);
   float f;
-  const int scaled = *sc.scaled;
-  const double ps = sc.psum[lane];
-  if (!uni(scaled)) return false;
-  const double total = wave_sum_f64(ps);
+  const int scaled = *sc.scaled;  // looked at once the sums have arrived too
+  const double ps = sc.psum[lane], total = wave_sum_f64(ps);
   const double slack = sum_slack(total, n);
   auto total_sure = [&](float* v) {  // (float)total
     return sure_float(total, slack, v) ||
            (uni(exact_sum(total, least_prob(sc, pc, seg, sm))) && sure_float(total, 0.0, v));
   };
+  if (!uni(scaled)) return false;
   uint64_t g = rng;
   if (p.top_p >= 1.0f && (p.top_k <= 0 || p.top_k >= n)) {
     // in index order: the list, then the entry the walk ends at
